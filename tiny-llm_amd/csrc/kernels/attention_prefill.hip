@@ -1,6 +1,5 @@
 // Prefill attention for gfx950: causal attention of a block of new query
-// tokens over a KV view, GQA, on MFMA; plus the reference's softmax and
-// attention-weights kernels.
+// tokens over a KV view, GQA, on MFMA.
 //
 // Per query token i of a sequence whose new tokens start at position p0 and
 // query head h (kv head g = h / G):
@@ -154,14 +153,6 @@ __device__ __forceinline__ uint4 ld16(const char *p) { return *reinterpret_cast<
 // the register file.
 template <int D>
 constexpr int kQueryGroups = D <= 128 ? 2 : 1;
-
-// Rounds x to fp32 in a register before whatever consumes it: keeps the
-// compiler from folding a multiply into the fp16 conversion that follows
-// (v_fma_mixlo_f16 rounds once, the reference's __float2half(a * b) twice).
-__device__ __forceinline__ float materialize(float x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
 
 template <int D, int G, bool PAGED, int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void attn_prefill_kernel(PrefillArgs a) {
@@ -517,51 +508,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 12
     }
 }
 
-// softmax_kernel (attention.cu:288-343): one workgroup per row.
-__global__ __launch_bounds__(256) void softmax_kernel(const __half *in, __half *out, int S) {
-    __shared__ float red[8];
-    const __half *x = in + (int64_t)blockIdx.x * S;
-    __half       *y = out + (int64_t)blockIdx.x * S;
-    const int     tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float         m = -FLT_MAX;
-    for (int i = tid; i < S; i += 256) m = fmaxf(m, __half2float(x[i]));
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if (lane == 0) red[wave] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    constexpr float kLog2e = 1.4426950408889634f;
-    float           sum = 0.0f;
-    for (int i = tid; i < S; i += 256) sum += exp2f((__half2float(x[i]) - m) * kLog2e);
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-    if (lane == 0) red[4 + wave] = sum;
-    __syncthreads();
-    sum = (red[4] + red[5]) + (red[6] + red[7]);
-    const float inv = 1.0f / (sum + 1e-6f);
-    for (int i = tid; i < S; i += 256)
-        y[i] = __float2half(materialize(exp2f((__half2float(x[i]) - m) * kLog2e) * inv));
-}
-
-// get_attention_weights_kernel (attention.cu:240-268): one thread per
-// (query, key) score, the reference's sequential fmaf order over d, then
-// score * scale rounded to fp32 and to fp16.
-__global__ __launch_bounds__(256) void attention_weights_kernel(const __half *q, const __half *k,
-                                                                __half *w, float scale, int H,
-                                                                int Lq, int Lk, int D, int causal) {
-    const int     i = blockIdx.y, bh = blockIdx.z;
-    const int     p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= Lk) return;
-    const __half *qr = q + ((int64_t)bh * Lq + i) * D;
-    const __half *kr = k + ((int64_t)bh * Lk + p) * D;
-    float         v = 0.0f;
-    if (!(causal && p > i)) {
-        float score = 0.0f;
-        for (int d = 0; d < D; ++d) score = fmaf(__half2float(qr[d]), __half2float(kr[d]), score);
-        v = materialize(score * scale);
-    }
-    w[((int64_t)bh * Lq + i) * Lk + p] = __float2half(v);
-    (void)H;
-}
-
 template <int D, int G, int NW>
 void launch_dgw(const PrefillArgs &a, int grid, bool paged, hipStream_t stream) {
     if (paged)
@@ -722,21 +668,6 @@ void launch_attn_prefill(const PrefillLaunch &p, const KvView &kv, int Hq, int H
     }
     HIP_CHECK(hipGetLastError());
     profile_end(KernelId::AttnPrefill, stream);
-}
-
-void launch_softmax(const __half *in, __half *out, int rows, int S, hipStream_t stream) {
-    if (rows <= 0 || S <= 0) return;
-    hipLaunchKernelGGL(softmax_kernel, dim3(rows), dim3(256), 0, stream, in, out, S);
-    HIP_CHECK(hipGetLastError());
-}
-
-void launch_attention_weights(const __half *q, const __half *k, __half *w, float scale, int B,
-                              int H, int Lq, int Lk, int D, bool causal, hipStream_t stream) {
-    if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= 0 || D <= 0) return;
-    dim3 grid((unsigned)((Lk + 255) / 256), (unsigned)Lq, (unsigned)(B * H));
-    hipLaunchKernelGGL(attention_weights_kernel, grid, dim3(256), 0, stream, q, k, w, scale, H, Lq,
-                       Lk, D, causal ? 1 : 0);
-    HIP_CHECK(hipGetLastError());
 }
 
 } // namespace detail

@@ -1,0 +1,121 @@
+"""GPU: the prompt-sized W8A16 kernel (more than 64 rows) at the edges of its
+tiles, K halves and scale groups, against the product in 64 bits.  Bar: 1e-3
+normwise per row, the W8A16 bar (fp16 rounding of an output leaves 2^-11)."""
+import numpy as np
+import pytest
+
+from devutil import empty_dev, stream, to_dev, to_dev_raw, to_host
+from test_gpu_w8a16 import TOL, _cache, operands, packed_dev, rows_close
+
+pytestmark = pytest.mark.gpu
+
+
+def both(tl, dx, w, ds, M, N, K, gs):
+    """fp16(x @ W) from the row-major weights and from the packed ones."""
+    out, dw = empty_dev((M, N)), to_dev_raw(w)
+    tl.w8a16_matmul(dx.data_ptr(), dw.data_ptr(), ds.data_ptr(), out.data_ptr(), M, N, K, gs, stream())
+    dh, dp = to_dev(np.zeros((M, N), np.uint16)), packed_dev(tl, w)
+    tl.w8a16_matmul_residual(dx.data_ptr(), dp.data_ptr(), ds.data_ptr(), dh.data_ptr(), M, N, K, gs, stream(),
+                             packed=True)
+    return to_host(out), to_host(dh)
+
+
+def product(x, w, s, K, gs):
+    """x @ dequant(w, s) in 64 bits (the outputs here are too many for the oracle)."""
+    sc = np.repeat(s.view(np.float16).astype(np.float64).reshape(-1, w.shape[1]), gs, axis=0)[:K]
+    return x.view(np.float16).astype(np.float64) @ (w.astype(np.float64) * sc)
+
+
+@pytest.mark.parametrize("M,N,K,gs", [
+    (65, 36304, 32, 32),     # one row over, one k step: no chunk at all, a column tail
+    (127, 18608, 64, 64),    # one chunk of two steps: the second K half is empty
+    (128, 18432, 96, 32),    # full tiles, an unpaired last step
+    (129, 18304, 160, 128),  # one row over, a partial last scale group
+    (257, 9232, 128, 32),    # two groups per chunk, a column tail
+    (320, 7408, 288, 64),    # several row tiles, K % 64 == 32 inside a group
+    (200, 6560, 2080, 512),  # few rows with a long K; groups across chunks and the K halves' boundary
+    (2390, 1008, 192, 256),  # more row tiles than a panel, a group longer than K
+    (9250, 256, 64, 32),     # one column tile
+    (600, 8192, 1056, 128),  # the widest tiles' other shapes
+])
+def test_w8a16_tile_edges(tl, orc, M, N, K, gs):
+    rng = np.random.default_rng(M + 3 * N + 7 * K + gs)
+    x, w, s = operands(orc, rng, M, N, K, gs)
+    ref = product(x, w, s, K, gs)
+    got, got_p = both(tl, to_dev(x), w, to_dev(s), M, N, K, gs)
+    assert rows_close(got, ref) <= TOL
+    # zero residual: fp16(0 + v) drops only the sign of a -0
+    assert np.array_equal(np.where(got == 0x8000, 0, got), got_p)
+
+
+def test_w8a16_tile_scales(tl, orc):
+    """Zero scales (whole columns, first, middle and last groups), negative and
+    subnormal ones, and scales far apart."""
+    M, N, K, gs = 96, 24592, 512, 64
+    rng = np.random.default_rng(8)
+    x, w, s = operands(orc, rng, M, N, K, gs)
+    f = s.view(np.float16).reshape(K // gs, N)
+    f[:, 3] = 0
+    f[0, 5] = f[1, 5] = f[4, 6] = f[-1, 7] = f[3, 17:40] = 0
+    f[2, 8] = -f[2, 8]
+    f[1, 9], f[5, 10] = 6e-8, 3e-6   # subnormal
+    # (64 products of |x| < 5, |w| <= 128, x of unit variance: |sum| < 6 * 128 * 8, times 5 below 65504)
+    f[2, 11], f[3, 11] = 5.0, 1e-5
+    f[6, 12] = -0.0
+    ref = product(x, w, s, K, gs)
+    got, got_p = both(tl, to_dev(x), w, to_dev(s), M, N, K, gs)
+    g = got.view(np.float16).astype(np.float64)
+    cols = np.abs(g - ref).max(axis=0) / np.maximum(np.abs(ref).max(axis=0), 1e-30)
+    assert np.all(g[:, 3] == 0) and cols.max() <= TOL  # per column: small columns count as much
+    assert np.array_equal(np.where(got == 0x8000, 0, got), got_p)
+
+
+def test_w8a16_tile_unaligned_output(tl, orc):
+    """An output base two bytes past a 16-byte boundary: element stores, and
+    nothing outside the matrix is written."""
+    M, N, K, gs = 300, 8208, 128, 128
+    rng = np.random.default_rng(4)
+    x, w, s = operands(orc, rng, M, N, K, gs)
+    dx, dw, ds = to_dev(x), to_dev_raw(w), to_dev(s)
+    out, off = empty_dev((M, N)), to_dev(np.full(M * N + 2, 0x3555, np.uint16))
+    tl.w8a16_matmul(dx.data_ptr(), dw.data_ptr(), ds.data_ptr(), out.data_ptr(), M, N, K, gs, stream())
+    tl.w8a16_matmul(dx.data_ptr(), dw.data_ptr(), ds.data_ptr(), off.data_ptr() + 2, M, N, K, gs, stream())
+    got = to_host(off)
+    assert np.array_equal(got[1:-1], to_host(out).reshape(-1)) and got[0] == got[-1] == 0x3555
+
+
+@pytest.mark.parametrize("paged,B,Hkv,D", [
+    (False, 130, 2, 64),    # all columns to the split-K kernel
+    (True, 310, 8, 256),    # q to the tile kernel, k and v to the split-K one
+    (False, 1200, 8, 256),  # all to the tile kernel
+    (True, 1200, 8, 256),
+])
+def test_project_large_batch_equals_products(tl, orc, paged, B, Hkv, D):
+    """The fused projection's cache bytes and q_out are those of the separate
+    products, whatever columns share the call."""
+    from devutil import read_dev
+    rng = np.random.default_rng(31 + paged)
+    G, hidden, gs = 4, 320, 64
+    row, Hq = Hkv * D, Hkv * G
+    lens = [int(v) for v in rng.integers(1, 12, size=B)]
+    g, _, ids, _k = _cache(tl, orc, np.random.default_rng(6), 1, Hkv, D, 16, lens, paged)
+    g2, _, ids2, _k2 = _cache(tl, orc, np.random.default_rng(6), 1, Hkv, D, 16, lens, paged)
+    x = orc.f2h(rng.standard_normal((B, hidden)).astype(np.float32))
+    ws = [operands(orc, rng, 1, n, hidden, gs)[1:] for n in (row, row, Hq * D)]
+    dx = to_dev(x)
+    dev = [(to_dev_raw(w), to_dev(s)) for w, s in ws]
+    (dwk, dsk), (dwv, dsv), (dwq, dsq) = dev
+    batch, q_out = tl.DecodeBatch(g, B, Hq), empty_dev((B, Hq * D))
+    batch.prepare(ids, stream())
+    batch.project(0, dx.data_ptr(), hidden, gs, dwk.data_ptr(), dsk.data_ptr(), dwv.data_ptr(), dsv.data_ptr(),
+                  dwq.data_ptr(), dsq.data_ptr(), q_out.data_ptr(), stream())
+    outs = [empty_dev((B, n)) for n in (row, row, Hq * D)]
+    for (dw, ds), o in zip(dev, outs):
+        tl.w8a16_matmul(dx.data_ptr(), dw.data_ptr(), ds.data_ptr(), o.data_ptr(), B, o.shape[1], hidden, gs, stream())
+    batch2 = tl.DecodeBatch(g2, B, Hq)
+    batch2.prepare(ids2, stream())
+    batch2.append(0, 1, outs[0].data_ptr(), outs[1].data_ptr(), stream())
+    n = g.slot_bytes() // 2 * (B + 1)
+    assert np.array_equal(read_dev(g.pool(), n), read_dev(g2.pool(), n))
+    assert np.array_equal(to_host(q_out), to_host(outs[2]))
+    assert rows_close(to_host(q_out), product(x, *ws[2], hidden, gs)) <= TOL

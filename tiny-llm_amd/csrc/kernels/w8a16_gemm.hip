@@ -5,7 +5,7 @@
 // [ceil(K/gs)][N] fp16.
 //
 // MFMA path (K % 32 == 0, gs in {32, 64, 128, 256, 512}, every segment's
-// N % 16 == 0), two kernels, each for both weight layouts (packed: the
+// N % 16 == 0), three kernels, each for both weight layouts (packed: the
 // launch_w8a16_pack layout, B fragments of 8 bytes per lane, two k steps per
 // 16-byte lane load; reference:
 // [K][N] row-major, staged in LDS and read as B fragments by the transposing
@@ -17,6 +17,9 @@
 //   w8a16_dec_kernel (M <= 64, K a multiple of 128 up to 4096: the decode
 //     projections): one launch over the whole of K, no partials (described
 //     at the kernel).
+//   w8a16_tile_kernel (prompt-sized outputs, tile_ok): one workgroup = 8 waves
+//     = up to a 128 x 256 output tile over the whole of K (described at the
+//     kernel).
 //   w8a16_sk_kernel (every other MFMA shape): one workgroup = 4 waves = a
 //     64x64 output tile over one K split; wave w takes every fourth group of
 //     4 k steps for the whole tile; x staged two k steps at a time in the
@@ -25,8 +28,9 @@
 //     writes fp32 partials and w8a16_reduce_kernel sums the splits in split
 //     order and applies it.
 //
-// The summation order of an output element depends on (M, K) only -- never
-// on which other weight matrices share the launch -- so results are
+// The summation order of an output element depends on (M, K), the group size and
+// its own matrix's columns only -- never on which other weight matrices share the
+// call -- so results are
 // deterministic and the fused projection equals the unfused products.
 //
 // Generic path (any shape): one thread per output, the reference formula
@@ -67,6 +71,7 @@ constexpr int kWaitLgkm0 = 0xC07F; // s_waitcnt lgkmcnt(0)
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float    f32x4 __attribute__((ext_vector_type(4)));
 typedef int      v2i32 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct GemmArgs {
@@ -818,6 +823,468 @@ __global__ __launch_bounds__(512, 1) void w8a16_dec_kernel(DecArgs a) {
     }
 }
 
+// The epilogue of eight consecutive columns n..n+7 of one segment (n % 8 == 0)
+// whose fp16 results are v.  vec: every output, residual and cache row piece
+// is 16-byte aligned; otherwise element by element.
+__device__ __forceinline__ void epilogue8(const GemmArgs &a, int si, int m, int n, uint4 v, int vec) {
+    const W8A16Seg &sg = a.seg[si];
+    int64_t         off = (int64_t)m * sg.ld + n;
+    if (sg.kind == kEpiCache) {
+        const CacheRows &c = a.cache;
+        const int        row = c.seq_row[m];
+        const int        t = c.wpos[m];
+        const int64_t    blk = c.block_table ? (int64_t)c.block_table[(int64_t)row * c.bt_stride + (t >> c.log2_blk)] : row;
+        off = blk * c.blk_stride + (int64_t)(t & ((1 << c.log2_blk) - 1)) * c.tok_stride + n;
+    }
+    __half o[8];
+    __builtin_memcpy(o, &v, 16);
+    if (sg.kind == kEpiResidual) { // fp16(f(res) + f(fp16(acc))), element by element
+        __half r[8];
+        if (vec) {
+            const uint4 rv = *reinterpret_cast<const uint4 *>(sg.res + off);
+            __builtin_memcpy(r, &rv, 16);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) r[i] = sg.res[off + i];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = __float2half(h2f(r[i]) + h2f(o[i]));
+    }
+    if (vec) {
+        __builtin_memcpy(&v, o, 16);
+        *reinterpret_cast<uint4 *>(sg.out + off) = v;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sg.out[off + i] = o[i];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Prompt-sized M: w8a16_tile_kernel, bound by the matrix rate.
+//
+// A workgroup of 8 waves owns a (16 RB) x (64 CB) output tile.  Its waves are
+// four column groups of 16 CB columns times two halves of K (64-row chunks of
+// K, the first half of them to waves 0-3): each wave multiplies all rows of the
+// tile by its own columns over its half, so that a weight is converted to fp16
+// by one wave only, two waves share a SIMD, and an x tile in LDS feeds four
+// waves.  At RB = 8, CB = 4 a chunk reads 16 KB of x from LDS and 4 KB of
+// weights per wave for 64 MFMAs: half the LDS rate at the full matrix rate.
+// x comes by the LDS DMA load into double-buffered tiles (rows of 128 bytes,
+// 16-byte piece c of row r in slot c ^ f(r) as in the split-K kernel), the
+// next chunk's during this one's products; packed weights load straight into
+// fragments one chunk ahead, row-major ones pass through the wave's LDS stage
+// and the transposing read.
+//
+// The products accumulate in units of the current scale group: T holds
+// (sum so far) / s, the MFMAs add to it directly, and where a group ends T is
+// multiplied by s / s_next -- one VALU operation per output and group, like
+// folding a separate product into an accumulator, but with one register per
+// output instead of two, which is what lets a wave hold 128 x 64 outputs.  A
+// zero scale keeps the last nonzero one and zeroes its columns' weights
+// instead.  At the end T * s of the two K halves are added through LDS.
+//
+// The order of an output's sum depends on K and the group size only, never on
+// the tile shape, the columns or the other segments.
+// 2048 x 4096 x 4096, group 128: 75-79 us row-major (870-920 TFLOP/s), 71-74
+// packed, against 113 / 108 for the split-K kernel; 585 x 8192 x 8192 97
+// packed, 125 before.  Timing-only copies (2048, packed): no folds 67, nor
+// conversions 62, nor MFMAs 42, loads and barriers alone 38: the VALU work and
+// the MFMAs overlap little, within a wave (conversions scheduled between MFMAs
+// measured level) or between the two waves of a SIMD.
+// Column tiles never span segments.  XCDs (workgroup index modulo 8) take
+// contiguous ranges of tiles, numbered down panels of a few row tiles, so
+// that the workgroups of an XCD share x rows and weight columns in its L2.
+struct TileArgs {
+    GemmArgs g;
+    int      log2_spg; // log2 of k steps (32 rows) per scale group
+    int      rtiles, ctiles, panel;
+    int      tpx; // tiles per XCD
+    int      vec; // outputs may be stored 16 bytes at a time
+};
+
+// x tiles and weight slots, one being multiplied and the others on the way: as
+// many as the registers (weights) and LDS hold.
+constexpr int tile_buffers(int RB, int CB) { return RB * CB > 24 ? 2 : RB == 8 ? 3 : 4; }
+
+// Rotation of the row-major weight tile: 16-byte piece p of row r sits in slot
+// (p + tile_rot(r)) % (4 CB), so that the 8 rows that a transposing read
+// touches (one piece each, rows 64 CB bytes apart) fall on distinct banks.
+template <int CB> __device__ __forceinline__ int tile_rot(int r) {
+    return CB == 4 ? (r & 7) : CB == 3 ? ((r >> 2) & 1) : ((r >> 1) & 3);
+}
+
+// The transposing reads of a chunk's two k steps (32 rows of 64 CB bytes
+// apart) for CB column blocks, complete when it returns.  In asm, because the
+// compiler waits for every outstanding LDS DMA before the builtin's read.
+template <int CB> __device__ __forceinline__ void read_tr(const uint32_t (&ad)[CB], uint2 (&raw)[2][CB]) {
+    u32x2 o[2][4];
+    if constexpr (CB == 4)
+        asm volatile("ds_read_b64_tr_b8 %0, %8\n\tds_read_b64_tr_b8 %1, %9\n\t"
+                     "ds_read_b64_tr_b8 %2, %10\n\tds_read_b64_tr_b8 %3, %11\n\t"
+                     "ds_read_b64_tr_b8 %4, %8 offset:8192\n\tds_read_b64_tr_b8 %5, %9 offset:8192\n\t"
+                     "ds_read_b64_tr_b8 %6, %10 offset:8192\n\tds_read_b64_tr_b8 %7, %11 offset:8192\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(o[0][0]), "=&v"(o[0][1]), "=&v"(o[0][2]), "=&v"(o[0][3]), "=&v"(o[1][0]), "=&v"(o[1][1]),
+                       "=&v"(o[1][2]), "=&v"(o[1][3])
+                     : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3])
+                     : "memory");
+    else if constexpr (CB == 3)
+        asm volatile("ds_read_b64_tr_b8 %0, %6\n\tds_read_b64_tr_b8 %1, %7\n\tds_read_b64_tr_b8 %2, %8\n\t"
+                     "ds_read_b64_tr_b8 %3, %6 offset:6144\n\tds_read_b64_tr_b8 %4, %7 offset:6144\n\t"
+                     "ds_read_b64_tr_b8 %5, %8 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(o[0][0]), "=&v"(o[0][1]), "=&v"(o[0][2]), "=&v"(o[1][0]), "=&v"(o[1][1]), "=&v"(o[1][2])
+                     : "v"(ad[0]), "v"(ad[1]), "v"(ad[2])
+                     : "memory");
+    else
+        asm volatile("ds_read_b64_tr_b8 %0, %4\n\tds_read_b64_tr_b8 %1, %5\n\t"
+                     "ds_read_b64_tr_b8 %2, %4 offset:4096\n\tds_read_b64_tr_b8 %3, %5 offset:4096\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(o[0][0]), "=&v"(o[0][1]), "=&v"(o[1][0]), "=&v"(o[1][1])
+                     : "v"(ad[0]), "v"(ad[1])
+                     : "memory");
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) raw[s][cb] = make_uint2(o[s][cb][0], o[s][cb][1]);
+}
+
+template <int RB, int CB, bool PACKED, bool FINE>
+__global__ __launch_bounds__(512, 2) void w8a16_tile_kernel(TileArgs ta) {
+    static_assert(RB == 4 || RB == 8, "row blocks");
+    static_assert(CB >= 2 && CB <= 4, "column blocks per wave");
+    const GemmArgs &a = ta.g;
+    constexpr int   XH = RB * 16 * 64;             // halves of one x tile (a chunk of one K half)
+    constexpr int   BN = 64 * CB;                  // columns of the tile
+    constexpr int   WT = PACKED ? 16 : 2 * 64 * BN; // bytes of a row-major weight tile of both K halves
+    // x tiles, as arrays of their own: the compiler's wait counts tell the loads
+    // into one from the reads of another.
+    constexpr int NBUF = tile_buffers(RB, CB);
+    __shared__ __align__(16) uint16_t xs0[2 * XH], xs1[2 * XH];
+    __shared__ __align__(16) uint16_t xs2[NBUF > 2 ? 2 * XH : 8], xs3[NBUF > 3 ? 2 * XH : 8];
+    __shared__ __align__(16) uint8_t  wt[2 * WT];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kh = wave >> 2, cg = wave & 3;
+    // Tile of this workgroup: panels of `panel` row tiles, in each the columns
+    // one after the other, row tiles fastest.
+    const int t = (int)(blockIdx.x & 7) * ta.tpx + (int)(blockIdx.x >> 3);
+    if (t >= ta.rtiles * ta.ctiles) return; // uniform for the workgroup
+    const int pan = t / (ta.panel * ta.ctiles);
+    const int inp = t - pan * ta.panel * ta.ctiles;
+    const int ph = min(ta.panel, ta.rtiles - pan * ta.panel);
+    const int m0 = (pan * ta.panel + inp % ph) * RB * 16;
+    int       ct = inp / ph, si = 0;
+    while (si + 1 < a.nseg && ct >= (a.seg[si].n + BN - 1) / BN) {
+        ct -= (a.seg[si].n + BN - 1) / BN;
+        ++si;
+    }
+    // Fields of the arguments that the loop needs, in registers: the barrier
+    // below is a memory clobber, behind which the compiler would reload them.
+    const int             M = a.M, lspg = ta.log2_spg;
+    const int             wn = a.seg[si].n;
+    const int8_t *const   sw = a.seg[si].w;
+    const uint16_t *const ss = reinterpret_cast<const uint16_t *>(a.seg[si].s);
+    const int             c0 = ct * BN + cg * 16 * CB; // the wave's first column
+    const int             ksteps = a.K >> 5;
+    const int             nchunks = ksteps >> 1; // chunks of two k steps (a last single step comes after the loop)
+    const int             half = (nchunks + 1) >> 1;
+    const int             cbeg = kh ? half : 0;
+    const int             cnt = kh ? nchunks - half : half;
+
+    // x: DMA u of the wave brings rows 8 (cg RB / 2 + u) + lane / 8 of the tile.
+    constexpr int NX = RB / 2;
+    uint32_t      xoff[NX]; // lane byte offsets into the row tile
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+        const int r = 8 * (cg * NX + u) + (lane >> 3);
+        xoff[u] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)a.ldx * 2u +
+                  16u * (uint32_t)((lane & 7) ^ (lane >> 3) ^ ((r >> 3) & 1));
+    }
+    const char *const xbase = reinterpret_cast<const char *>(a.x + (int64_t)m0 * a.ldx);
+    // (chunks past the end re-read the last one; they are never multiplied)
+    auto issue_x = [&](int j, uint16_t *buf) __attribute__((always_inline)) {
+        const char *src = xbase + (int64_t)min(cbeg + j, nchunks - 1) * 128;
+#pragma unroll
+        for (int u = 0; u < NX; ++u)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + xoff[u]),
+                                             (__attribute__((address_space(3))) void *)(buf + kh * XH + (cg * NX + u) * 512),
+                                             16, 0, 0);
+    };
+    // Weights and scales of chunk j, in registers.
+    const int8_t *wp[CB];
+    uint32_t      scol[CB];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+        const int nb = min((c0 >> 4) + cb, (wn >> 4) - 1);
+        wp[cb] = sw + (int64_t)nb * ksteps * 512;
+        scol[cb] = (uint32_t)(16 * nb + (lane & 15));
+    }
+    // Row-major: the four waves of a K half bring the tile's 64 rows x BN columns
+    // of a chunk, thread by thread 16 bytes of slot 256 q + thread.
+    const int th = cg * 64 + lane;
+    uint32_t  woff[CB];
+    if constexpr (!PACKED) {
+#pragma unroll
+        for (int q = 0; q < CB; ++q) {
+            const int s = q * 256 + th, r = s / (4 * CB);
+            const int p = (s % (4 * CB) + 4 * CB - tile_rot<CB>(r)) % (4 * CB);
+            woff[q] = (uint32_t)r * (uint32_t)wn + (uint32_t)min(ct * BN + 16 * p, wn - 16);
+        }
+    }
+    constexpr int NS = FINE ? 2 : 1; // scale groups of a chunk: two for a group size of 32
+    struct WSlot {
+        u32x4    w[CB];
+        uint16_t s[NS][CB];
+    };
+    auto load_w = [&](WSlot &sl, int j) __attribute__((always_inline)) {
+        const int ck = min(cbeg + j, nchunks - 1);
+        if constexpr (PACKED) {
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+                sl.w[cb] = *reinterpret_cast<const u32x4 *>(wp[cb] + (int64_t)ck * 1024 + 16 * lane);
+        } else {
+            const int8_t *src = sw + (int64_t)ck * 64 * wn;
+#pragma unroll
+            for (int q = 0; q < CB; ++q) sl.w[q] = *reinterpret_cast<const u32x4 *>(src + woff[q]);
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const uint16_t *sp = ss + (int64_t)((2 * ck + s) >> lspg) * wn;
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) sl.s[s][cb] = sp[scol[cb]];
+        }
+    };
+    // Row-major: into weight tile j % 2.  In asm, because the compiler waits for
+    // every outstanding LDS DMA before an LDS store of its own; the step waits
+    // for these stores itself.
+    const uint32_t wlds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)wt;
+    auto store_w = [&](const WSlot &sl, int j) __attribute__((always_inline)) {
+        if constexpr (!PACKED) {
+            const uint32_t dst = wlds + (uint32_t)((j & 1) * WT + kh * (WT / 2) + th * 16);
+#pragma unroll
+            for (int q = 0; q < CB; ++q)
+                asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(dst), "v"(sl.w[q]), "n"(q * 4096) : "memory");
+        }
+    };
+
+    f32x4 acc[RB][CB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float s_cur[CB];
+    bool  zero[CB]; // the scale of this lane's column is zero in the current group
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+        s_cur[cb] = 1.0f;
+        zero[cb] = false;
+    }
+    const int fr = (lane & 7) ^ ((lane >> 3) & 1); // f of the lane's fragment rows
+    // Row-major: lane i of a 16-lane group q names 8 bytes of row 8q + i/2 (the
+    // rotation is the same 32 rows on), columns 16 cb + 8 (i % 2).
+    uint32_t trl[CB];
+    if constexpr (!PACKED) {
+        const int i = lane & 15, r = 8 * (lane >> 4) + (i >> 1);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+            trl[cb] = (uint32_t)((r * 4 * CB + (cg * CB + cb + tile_rot<CB>(r)) % (4 * CB)) * 16 + 8 * (i & 1));
+    }
+    // A scale group begins: T, still 0 before the first, goes over to its units.
+    auto new_group = [&](const uint16_t(&sc)[CB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            const float sn = h2f(__builtin_bit_cast(__half, sc[cb]));
+            zero[cb] = sn == 0.0f;
+            const float se = zero[cb] ? s_cur[cb] : sn;
+            const float ratio = s_cur[cb] / se;
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[rb][cb][i] *= ratio;
+            s_cur[cb] = se;
+        }
+    };
+    auto multiply = [&](const f16x8(&xa)[RB], uint2 raw, int cb) __attribute__((always_inline)) {
+        const uint32_t none = PACKED ? 0x80808080u : 0u;
+        raw.x = zero[cb] ? none : raw.x;
+        raw.y = zero[cb] ? none : raw.y;
+        const uint2 lo = w8x4_to_f16x4<PACKED>(raw.x), hi = w8x4_to_f16x4<PACKED>(raw.y);
+        const f16x8 bop = __builtin_bit_cast(f16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+            acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[rb], bop, acc[rb][cb], 0, 0, 0);
+    };
+    auto read_x = [&](const uint16_t *buf, int s, f16x8(&xa)[RB]) __attribute__((always_inline)) {
+        const uint16_t *xt = buf + kh * XH + (lane & 15) * 64;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+            xa[rb] = *reinterpret_cast<const f16x8 *>(xt + rb * 1024 + 8 * ((4 * s + (lane >> 4)) ^ fr));
+    };
+    auto compute = [&](const uint16_t *buf, const WSlot &sl, int j) __attribute__((always_inline)) {
+        if (FINE || j == 0 || ((2 * (cbeg + j)) & ((1 << lspg) - 1)) == 0) new_group(sl.s[0]);
+        uint2 raw[2][CB];
+        if constexpr (PACKED) {
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                raw[0][cb] = make_uint2(sl.w[cb][0], sl.w[cb][1]);
+                raw[1][cb] = make_uint2(sl.w[cb][2], sl.w[cb][3]);
+            }
+        } else {
+            const uint32_t base = wlds + (uint32_t)((j & 1) * WT + kh * (WT / 2));
+            uint32_t       ad[CB];
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) ad[cb] = base + trl[cb];
+            read_tr<CB>(ad, raw);
+        }
+        f16x8 xa[RB], xb[RB];
+        read_x(buf, 0, xa);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) multiply(xa, raw[0][cb], cb);
+        read_x(buf, 1, xb);
+        if constexpr (FINE) new_group(sl.s[NS - 1]);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) multiply(xb, raw[1][cb], cb);
+        
+    };
+    // Chunk j from `cur` while chunks j + 1 .. j + DIST are on the way, the last
+    // of them issued here into the slot that chunk j - 1 freed (steps before 0
+    // only issue).  Every step issues the same number of loads, so the wait at
+    // its end -- chunk j + 1 has landed -- is a count.
+    constexpr int DIST = NBUF - 1;
+    constexpr int LATER = (DIST - 1) * (NX + CB + NS * CB); // loads of chunks j + 2 .. j + DIST
+    static_assert(LATER < 64, "vmcnt");
+    WSlot w0 = {}, w1 = {}, w2 = {}, w3 = {};
+    auto  step = [&](int j, uint16_t *cur, uint16_t *nxt, WSlot &wcur, WSlot &wone, WSlot &wnxt)
+                    __attribute__((always_inline)) {
+        load_w(wnxt, j + DIST);
+        issue_x(j + DIST, nxt);
+        if (j >= 0 && j < cnt) compute(cur, wcur, j);
+        // A bare barrier: a fenced one waits for every load.  The wait above it
+        // makes this wave's part of x tile j + 1 (and the weights stored after
+        // the wait) visible behind it; tile j has been read.
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (LATER & 15) | (LATER >> 4) << 14); // vmcnt(LATER)
+        store_w(wone, j + 1);
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // Whole rounds of the slots, also past the last chunk: with a branch around
+    // a step the compiler's wait counts would have to assume it was not taken.
+    if (nchunks > 0)
+        for (int j = -DIST; j < half; j += NBUF) {
+            if constexpr (NBUF == 2) {
+                step(j, xs1, xs0, w1, w0, w0);
+                step(j + 1, xs0, xs1, w0, w1, w1);
+            } else if constexpr (NBUF == 3) {
+                step(j, xs1, xs0, w1, w2, w0);
+                step(j + 1, xs2, xs1, w2, w0, w1);
+                step(j + 2, xs0, xs2, w0, w1, w2);
+            } else {
+                step(j, xs1, xs0, w1, w2, w0);
+                step(j + 1, xs2, xs1, w2, w3, w1);
+                step(j + 2, xs3, xs2, w3, w0, w2);
+                step(j + 3, xs0, xs3, w0, w1, w3);
+            }
+        }
+    __builtin_amdgcn_s_waitcnt(kWaitVm0); // the loads past the end have landed too
+    __syncthreads();
+    // A last unpaired k step, by the second K half, straight from memory.
+    if (kh && (ksteps & 1)) {
+        const int st = ksteps - 1;
+        uint16_t  sc[CB];
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) sc[cb] = ss[(int64_t)(st >> lspg) * wn + scol[cb]];
+        if (cnt == 0 || (st & ((1 << lspg) - 1)) == 0) new_group(sc);
+        f16x8 xa[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+            xa[rb] = *reinterpret_cast<const f16x8 *>(
+                xbase + ((int64_t)min(16 * rb + (lane & 15), M - 1 - m0) * a.ldx + 32 * st + 8 * (lane >> 4)) * 2);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            uint2 raw;
+            if constexpr (PACKED) {
+                raw = *reinterpret_cast<const uint2 *>(wp[cb] + (int64_t)nchunks * 1024 + 8 * lane);
+            } else {
+                uint32_t b[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    b[i] = (uint8_t)sw[(int64_t)(32 * st + 8 * (lane >> 4) + i) * wn + scol[cb]];
+                raw = make_uint2(b[0] | b[1] << 8 | b[2] << 16 | b[3] << 24, b[4] | b[5] << 8 | b[6] << 16 | b[7] << 24);
+            }
+            multiply(xa, raw, cb);
+        }
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[rb][cb][i] *= s_cur[cb];
+
+    // The two K halves: each wave hands the row blocks that the other half's
+    // wave finishes through the (free) x tiles: the first half of the row
+    // blocks is finished by waves 0-3, the second by waves 4-7.
+    constexpr int HB = RB / 2, QB = RB / 4; // row blocks per wave, and per array
+    auto ex = [&](int k) { // row block k of the passed half, this column group
+        float *b = reinterpret_cast<float *>(k < QB ? xs0 : xs1);
+        return b + ((cg * QB + k % QB) * CB * 64 + lane) * 4;
+    };
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+        if (kh != pass) { // give row blocks pass * HB ..
+#pragma unroll
+            for (int k = 0; k < HB; ++k)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+                    *reinterpret_cast<f32x4 *>(ex(k) + cb * 256) = acc[pass * HB + k][cb];
+        }
+        __syncthreads();
+        if (kh == pass) {
+#pragma unroll
+            for (int k = 0; k < HB; ++k)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    const f32x4 o = *reinterpret_cast<const f32x4 *>(ex(k) + cb * 256);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[pass * HB + k][cb][i] += o[i];
+                }
+        }
+        __syncthreads();
+    }
+    // Output: QB row blocks at a time through the wave's own part of the x
+    // tiles (rows of 16 CB halves, padded by 8), then 16-byte row pieces.
+    constexpr int OP = 16 * CB + 8, PPR = 2 * CB;
+    static_assert(4 * QB * 16 * OP <= 2 * XH, "the output stage fits an x tile pair");
+    uint16_t *st = (kh ? xs1 : xs0) + cg * QB * 16 * OP;
+#pragma unroll
+    for (int pq = 0; pq < 2; ++pq) {
+#pragma unroll
+        for (int k = 0; k < QB; ++k)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = kh ? acc[HB + pq * QB + k][cb][i] : acc[pq * QB + k][cb][i];
+                    st[(16 * k + 4 * (lane >> 4) + i) * OP + 16 * cb + (lane & 15)] =
+                        __builtin_bit_cast(uint16_t, __float2half(v));
+                }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int p = lane; p < QB * 16 * PPR; p += 64) {
+            const int r = p / PPR, c = 8 * (p - r * PPR);
+            const int m = m0 + 16 * (kh * HB + pq * QB) + r;
+            if (m < M && c0 + c < wn)
+                epilogue8(a, si, m, c0 + c, *reinterpret_cast<const uint4 *>(&st[r * OP + c]), ta.vec);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
 // Repacks W [K][N] int8 (K % 32 == 0, N % 16 == 0) into the B fragments of
 // v_mfma_f32_16x16x32_f16: lane l of the fragment of column block nb and k
 // step ks holds W[32 ks + 8 (l / 16) + j][16 nb + l % 16] ^ 0x80, j = 0..7 --
@@ -986,10 +1453,103 @@ DecPlan dec_plan(int M, int gs, const W8A16Seg *segs, int nseg) {
 }
 } // namespace
 
+namespace {
+// A segment of n columns goes to w8a16_tile_kernel by its own size, never by
+// what shares the call, so that the fused projection's bytes equal the separate
+// products'.  Its smallest tiles still walk K in steps of about 0.6 us, two
+// K halves at a time (27 us for K = 4096, however few the tiles), so it takes
+// the outputs that keep the split-K kernel busy longer than that.  Row-major /
+// packed us, split-K -> tile, K = 4096: 512 x 4096 32.2 / 32.0 -> 33.2 / 28.5
+// and 1536 x 1024 30.9 / 31.1 -> 32.3 / 27.6 (both left alone), 300 x 8192
+// 47.7 / 47.2 -> 45.2 / 37.2, 8192 x 256 45.1 / 47.3 -> 33.1 / 28.9; K = 14336:
+// 600 x 4096 138.6 / 127.1 -> 138.8 / 110.5.  Up to 256 rows the split-K kernel
+// also writes and sums partials when K is 2048 or more: 128 x 11008 40.2 / 39.3
+// -> 32.5 / 27.3, 256 x 8192 54.1 / 53.8 -> 32.9 / 28.8 (but K = 512, 192 x
+// 11008: 10.6 / 11.5 -> 12.1 / 11.2).
+bool tile_ok(int M, int n, int K) {
+    const int64_t outputs = (int64_t)M * n;
+    if (M <= 64) return false;
+    return outputs >= (M <= 256 && K >= 2048 ? 5LL << 18 : 9LL << 18);
+}
+
+// Plan of w8a16_tile_kernel: the tile shape with the least padded work in the
+// longest CU's share, (rounds of one workgroup per CU) x RB x CB, the larger
+// tile on a tie (its x and weight traffic per product is the lowest).
+struct TilePlan {
+    int rb = 8, cb = 4, rtiles = 0, ctiles = 0;
+};
+TilePlan tile_plan(int M, int gs, const W8A16Seg *segs, int nseg) {
+    TilePlan  best;
+    int64_t   cost = INT64_MAX;
+    const int cus = std::max(1, device_cus());
+    for (int rb = 8; rb >= 4; rb -= 4)
+        for (int cb = 4; cb >= 2; --cb) {
+            if (gs == 32 && rb == 8 && cb == 4) continue; // two scales per chunk do not fit its registers
+            TilePlan p;
+            p.rb = rb;
+            p.cb = cb;
+            p.rtiles = (M + 16 * rb - 1) / (16 * rb);
+            for (int i = 0; i < nseg; ++i) p.ctiles += (segs[i].n + 64 * cb - 1) / (64 * cb);
+            const int64_t rounds = ((int64_t)p.rtiles * p.ctiles + cus - 1) / cus;
+            if (rounds * rb * cb < cost) {
+                cost = rounds * rb * cb;
+                best = p;
+            }
+        }
+    return best;
+}
+
+void launch_tile(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
+    TileArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.g = g;
+    a.log2_spg = __builtin_ctz((unsigned)(gs / 32));
+    const TilePlan p = tile_plan(g.M, gs, g.seg, g.nseg);
+    a.rtiles = p.rtiles;
+    a.ctiles = p.ctiles;
+    a.panel = p.rtiles <= 6 ? p.rtiles : 4;
+    a.tpx = (p.rtiles * p.ctiles + 7) / 8;
+    uintptr_t low = 0;
+    for (int i = 0; i < g.nseg; ++i) {
+        low |= reinterpret_cast<uintptr_t>(g.seg[i].out);
+        if (g.seg[i].kind == kEpiResidual) low |= reinterpret_cast<uintptr_t>(g.seg[i].res);
+        low |= (uintptr_t)(g.seg[i].kind == kEpiCache ? g.cache.blk_stride | g.cache.tok_stride : g.seg[i].ld) * 2u;
+    }
+    a.vec = (low & 15u) == 0;
+    const dim3 grid((unsigned)(8 * a.tpx)), block(512);
+    profile_begin(KernelId::W8A16, stream);
+#define TL_W8_TILE(RB, CB, FINE)                                                                          \
+    do {                                                                                                  \
+        if (packed) hipLaunchKernelGGL((w8a16_tile_kernel<RB, CB, true, FINE>), grid, block, 0, stream, a); \
+        else hipLaunchKernelGGL((w8a16_tile_kernel<RB, CB, false, FINE>), grid, block, 0, stream, a);       \
+    } while (0)
+#define TL_W8_TILE_CB(RB, FINE)               \
+    do {                                      \
+        if (p.cb == 3) TL_W8_TILE(RB, 3, FINE); \
+        else TL_W8_TILE(RB, 2, FINE);           \
+    } while (0)
+    if (gs == 32) {
+        if (p.rb == 4 && p.cb == 4) TL_W8_TILE(4, 4, true);
+        else if (p.rb == 8) TL_W8_TILE_CB(8, true);
+        else TL_W8_TILE_CB(4, true);
+    } else if (p.cb == 4) {
+        if (p.rb == 8) TL_W8_TILE(8, 4, false);
+        else TL_W8_TILE(4, 4, false);
+    } else {
+        if (p.rb == 8) TL_W8_TILE_CB(8, false);
+        else TL_W8_TILE_CB(4, false);
+    }
+#undef TL_W8_TILE_CB
+#undef TL_W8_TILE
+    HIP_CHECK(hipGetLastError());
+    profile_end(KernelId::W8A16, stream);
+}
+} // namespace
+
 size_t w8a16_workspace_floats(int M, int K, int gs, const W8A16Seg *segs, int nseg) {
     if (!w8a16_mfma_ok(K, gs, segs, nseg) || dec_ok(M, K, segs, nseg)) return 0;
     int ntot = 0;
-    for (int i = 0; i < nseg; ++i) ntot += segs[i].n;
+    for (int i = 0; i < nseg; ++i) ntot += tile_ok(M, segs[i].n, K) ? 0 : segs[i].n;
     const int splits = split_plan(M, K, nullptr);
     return splits > 1 ? (size_t)splits * M * ntot : 0;
 }
@@ -1060,7 +1620,6 @@ void launch_w8a16(const __half *x, int64_t ldx, int M, int K, int gs, const W8A1
     for (int i = 0; i < nseg; ++i) {
         a.seg[i] = segs[i];
         a.col0[i + 1] = a.col0[i] + segs[i].n;
-        tiles += (segs[i].n + kBN - 1) / kBN;
         if (segs[i].kind == kEpiCache && !cache)
             throw std::invalid_argument("w8a16: cache epilogue without cache rows");
     }
@@ -1087,6 +1646,20 @@ void launch_w8a16(const __half *x, int64_t ldx, int M, int K, int gs, const W8A1
         launch_dec(a, gs, stream, packed);
         return;
     }
+    // Large segments to the tile kernel, the others to the split-K one.
+    GemmArgs big = a;
+    big.nseg = a.nseg = 0;
+    tiles = 0;
+    for (int i = 0; i < nseg; ++i) {
+        GemmArgs &to = tile_ok(M, segs[i].n, K) ? big : a;
+        to.seg[to.nseg] = segs[i];
+        to.col0[to.nseg + 1] = to.col0[to.nseg] + segs[i].n;
+        ++to.nseg;
+    }
+    if (big.nseg) launch_tile(big, gs, stream, packed);
+    if (!a.nseg) return;
+    for (int i = 0; i < a.nseg; ++i) tiles += (a.seg[i].n + kBN - 1) / kBN;
+    a.ntot = a.col0[a.nseg];
     const int mt = (M + kBM - 1) / kBM;
     const int splits = split_plan(M, K, &a.chunks_per_split);
     a.splits = splits;

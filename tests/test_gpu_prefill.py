@@ -358,3 +358,33 @@ def test_failed_prepare_leaves_an_empty_batch(tl):
     pb.commit()
     assert np.array_equal(read_dev(g.pool(), g.slot_bytes() // 2), before)
     assert g.getSeqLen(sid) == 100
+
+
+@pytest.mark.parametrize("paged", [False, True])
+def test_prefill_plans_in_arguments_and_in_memory_agree(tl, paged):
+    """A step whose work does not fit the kernel arguments (300 entries) gives
+    the bits of the same prompts in steps that do (100 entries each), and the
+    same cache."""
+    from devutil import read_dev
+    rng = np.random.default_rng(88)
+    H, D, Hq, M, n = 2, 64, 4, 32, 300
+    counts = [int(v) for v in rng.integers(1, 20, size=n)]
+    at = np.concatenate([[0], np.cumsum(counts)])
+    k, v = (to_dev(f16bits(rng, (int(at[-1]), H * D))) for _ in range(2))
+    q = to_dev(f16bits(rng, (int(at[-1]), Hq, D)))
+    outs, pools = [], []
+    for step in (n, 100):
+        g = tl.KVCacheManager(1, H, D, M, n, **(dict(block_tokens=16, num_blocks=2 * n) if paged else {}))
+        ids = [g.allocateSequence(M)[0] for _ in range(n)]
+        out = empty_dev(tuple(q.shape))
+        pb = tl.PrefillBatch(g, n, Hq)
+        for a in range(0, n, step):
+            pb.prepare(ids[a:a + step], counts[a:a + step], stream())
+            o, e = int(at[a]), 2  # bytes per half
+            pb.run(0, q.data_ptr() + o * Hq * D * e, k.data_ptr() + o * H * D * e, v.data_ptr() + o * H * D * e,
+                   out.data_ptr() + o * Hq * D * e, D ** -0.5, stream())
+            pb.commit()
+        outs.append(to_host(out))
+        halves = 2 * (2 * n + 1) * 16 * H * D if paged else n * 2 * M * H * D
+        pools.append(read_dev(g.pool(), halves))
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(pools[0], pools[1])

@@ -111,6 +111,7 @@ struct PrefillArgs {
     const __half       *new_v;
     int                 Hkv;
     float               scale_log2;
+    PrefillInline       inl; // used when inl.n_entries > 0
 };
 
 // Byte offsets of the token rows of one (cache row, kv head).
@@ -195,7 +196,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 12
     const int g = blockIdx.x - item * a.Hkv;
     int64_t   q_off;
     int       p0, n, row, qt, tok0 = 0;
-    if (a.work) { // one self-contained record: a single dependent load
+    if (a.inl.n_entries) {
+        const uint32_t it = (uint32_t)a.inl.w[4 * a.inl.n_entries + item];
+        const int      e = 4 * (int)(it >> 16);
+        p0 = a.inl.w[e];
+        n = a.inl.w[e + 1];
+        row = a.inl.w[e + 2];
+        tok0 = a.inl.w[e + 3];
+        qt = (int)(it & 0xFFFFu);
+        q_off = (int64_t)tok0 * a.q_tok;
+    } else if (a.work) { // one self-contained record: a single dependent load
         const int32_t *w = a.work + (int64_t)kPrefillItemWords * item;
         q_off = (int64_t)(((uint64_t)(uint32_t)w[1] << 32) | (uint32_t)w[0]);
         p0 = w[2];
@@ -594,19 +604,28 @@ int prefill_waves_uniform(int B, int S, int D, int G, int Hkv, int cus) {
     return waves_rule(D, (int64_t)B * nqt, (int64_t)B * keys, Hkv, cus);
 }
 
-void plan_prefill(const PrefillEntry *entries, int n, int D, int G, int waves, std::vector<int32_t> &work) {
+namespace {
+struct PrefillItem {
+    int64_t keys;
+    int32_t e, qt;
+};
+// (entry, query tile) items, most keys first.
+std::vector<PrefillItem> prefill_items(const PrefillEntry *entries, int n, int D, int G, int waves) {
     const int BQ = prefill_block_tokens(D, G, waves);
-    struct It {
-        int64_t keys;
-        int32_t e, qt;
-    };
-    std::vector<It> items;
+    std::vector<PrefillItem> items;
     for (int e = 0; e < n; ++e) {
         const int nqt = (entries[e].n + BQ - 1) / BQ;
         for (int qt = 0; qt < nqt; ++qt)
             items.push_back({(int64_t)entries[e].p0 + std::min(entries[e].n, (qt + 1) * BQ), e, qt});
     }
-    std::stable_sort(items.begin(), items.end(), [](const It &x, const It &y) { return x.keys > y.keys; });
+    std::stable_sort(items.begin(), items.end(),
+                     [](const PrefillItem &x, const PrefillItem &y) { return x.keys > y.keys; });
+    return items;
+}
+} // namespace
+
+void plan_prefill(const PrefillEntry *entries, int n, int D, int G, int waves, std::vector<int32_t> &work) {
+    const std::vector<PrefillItem> items = prefill_items(entries, n, D, G, waves);
     work.assign(kPrefillItemWords * items.size(), 0);
     for (size_t i = 0; i < items.size(); ++i) {
         const PrefillEntry &E = entries[items[i].e];
@@ -621,12 +640,31 @@ void plan_prefill(const PrefillEntry *entries, int n, int D, int G, int waves, s
     }
 }
 
+bool plan_prefill_inline(const PrefillEntry *entries, int n, int D, int G, int waves, PrefillInline &out) {
+    out.n_entries = out.n_items = 0;
+    const int BQ = prefill_block_tokens(D, G, waves);
+    int64_t   words = 4 * (int64_t)n;
+    for (int e = 0; e < n && words <= kPrefillInlineWords; ++e) words += (entries[e].n + (int64_t)BQ - 1) / BQ;
+    if (n <= 0 || words > kPrefillInlineWords) return false; // (so entries and tiles fit 16 bits)
+    const std::vector<PrefillItem> items = prefill_items(entries, n, D, G, waves);
+    for (int e = 0; e < n; ++e) {
+        out.w[4 * e] = entries[e].p0;
+        out.w[4 * e + 1] = entries[e].n;
+        out.w[4 * e + 2] = entries[e].row;
+        out.w[4 * e + 3] = entries[e].tok0;
+    }
+    for (size_t i = 0; i < items.size(); ++i) out.w[4 * n + (int)i] = items[i].e << 16 | items[i].qt;
+    out.n_entries = n;
+    out.n_items = (int)items.size();
+    return true;
+}
+
 void launch_attn_prefill(const PrefillLaunch &p, const KvView &kv, int Hq, int Hkv, int D,
                          float scale, hipStream_t stream) {
     const int G = Hq / Hkv;
     int       items, waves;
-    if (p.work) {
-        items = p.n_items;
+    if (p.work || p.inl) {
+        items = p.inl ? p.inl->n_items : p.n_items;
         waves = p.waves;
         if (waves != 4 && !(waves == 8 && D <= 128))
             throw std::invalid_argument("attention_prefill: the work list's waves per workgroup must be 4, or 8 "
@@ -647,7 +685,9 @@ void launch_attn_prefill(const PrefillLaunch &p, const KvView &kv, int Hq, int H
     a.q_entry = p.q_entry_stride;
     a.uniform_b = p.uniform_b;
     a.uniform_n = p.uniform_n;
-    if ((p.new_k != nullptr) != (p.new_v != nullptr) || (p.new_k && !p.work))
+    if (p.inl) a.inl = *p.inl;
+    else a.inl.n_entries = 0;
+    if ((p.new_k != nullptr) != (p.new_v != nullptr) || (p.new_k && !p.work && !p.inl))
         throw std::invalid_argument("attention_prefill: the fused append needs new_k, new_v and a work list");
     a.new_k = p.new_k;
     a.new_v = p.new_v;

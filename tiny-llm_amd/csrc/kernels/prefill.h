@@ -75,6 +75,22 @@ int  prefill_waves_setting();
 constexpr int kPrefillItemWords = 8;
 void plan_prefill(const PrefillEntry *entries, int n, int D, int G, int waves, std::vector<int32_t> &work);
 
+// The same work in the kernel arguments, so that a launch needs no host-to-device
+// copy: entries as {p0, n, row, tok0} (q_off is tok0 * q_tok_stride), then one
+// word per item, entry << 16 | query tile.  Two dependent scalar loads in place
+// of one, and in place of a copy of about 4 us in front of the kernel (prepare +
+// run, Llama-3-8B heads: 16 x 512 77.1 -> 73.0 us, 32 x 256 59.0 -> 54.2, one
+// prompt of 3 tokens 12.3 -> 8.5).
+constexpr int kPrefillInlineWords = 896;
+struct PrefillInline {
+    int32_t n_entries = 0;
+    int32_t n_items = 0;
+    int32_t w[kPrefillInlineWords];
+};
+// False when the entries and their items do not fit.  Entries must have q_off ==
+// tok0 * the launch's q_tok_stride.
+bool plan_prefill_inline(const PrefillEntry *entries, int n, int D, int G, int waves, PrefillInline &out);
+
 struct PrefillLaunch {
     const __half       *q = nullptr;
     __half             *out = nullptr;
@@ -85,7 +101,9 @@ struct PrefillLaunch {
     const int32_t      *work = nullptr;
     int                 n_items = 0;
     int                 waves = 0;
-    // ... or, with work == NULL, `uniform_b` entries b with p0 = 0,
+    // ... or the same in the kernel arguments (with `waves`) ...
+    const PrefillInline *inl = nullptr;
+    // ... or, with neither, `uniform_b` entries b with p0 = 0,
     // n = uniform_n, row = b and q_off = b * q_entry_stride (waves by
     // prefill_waves_uniform).
     int                 uniform_b = 0;
@@ -94,7 +112,7 @@ struct PrefillLaunch {
     // Largest p0 + n over the entries (the offset-width check of
     // contiguous rows).
     int                 max_keys = 0;
-    // Fused append (work-list launches only): the new tokens' K/V rows,
+    // Fused append (launches with a work list only): the new tokens' K/V rows,
     // [tokens][Hkv * D].  Keys at positions >= p0 are then read from here,
     // and the workgroup of each query tile writes its own tokens' rows of
     // its kv head into the cache -- the bytes of appendKV -- so the cache

@@ -30,6 +30,10 @@ struct W8A16Seg {
 struct CacheRows {
     const int32_t *seq_row = nullptr;
     const int32_t *wpos = nullptr;
+    // The same arrays in host memory: enough where w8a16_takes_dec says so (that
+    // kernel has them in its arguments), and seq_row / wpos may then be null.
+    const int32_t *host_row = nullptr;
+    const int32_t *host_wpos = nullptr;
     const int32_t *block_table = nullptr;
     int            bt_stride = 0;
     int            log2_blk = 30;
@@ -49,6 +53,9 @@ bool w8a16_mfma_ok(int K, int gs, const W8A16Seg *segs, int nseg);
 // MFMA shapes (e.g. M <= 64 with K = 14336) take the split-K pair and need it,
 // for the segments that w8a16_tile_kernel does not take.
 size_t w8a16_workspace_floats(int M, int K, int gs, const W8A16Seg *segs, int nseg);
+
+// True when launch_w8a16 will run w8a16_dec_kernel for these operands.
+bool w8a16_takes_dec(const __half *x, int64_t ldx, int M, int K, int gs, const W8A16Seg *segs, int nseg, bool packed);
 
 // out = x @ dequant(W_i, s_i) for each segment i, with its epilogue.  x [M][K]
 // fp16 at row pitch ldx; all pointers device; 16-byte alignment of x, W and

@@ -714,11 +714,10 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
     if (with_q && (!wq || !sq || !q_out))
         return Result<void>::err("DecodeBatch: wq, sq and q_out must be all set or all null");
     if (n_ == 0) return Result<void>::ok();
-    upload_device(stream);
-    const KvView v = mgr_.layerView(layer_idx, d_slot_);
+    const KvView v = mgr_.layerView(layer_idx, nullptr);
     detail::CacheRows rows;
-    rows.seq_row = d_slot_;
-    rows.wpos = d_wpos_;
+    rows.host_row = slot_.data();
+    rows.host_wpos = wpos_.data();
     rows.block_table = v.block_table;
     rows.bt_stride = v.bt_stride;
     rows.log2_blk = v.log2_blk;
@@ -745,6 +744,11 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
     if (packed && !detail::w8a16_mfma_ok(hidden, group_size, segs, nseg))
         return Result<void>::err("DecodeBatch: packed weights need hidden % 32 == 0 and group_size "
                                  "in {32, 64, 128, 256, 512}");
+    if (!detail::w8a16_takes_dec(x, hidden, n_, hidden, group_size, segs, nseg, packed)) {
+        upload_device(stream); // the other kernels read the rows from device memory
+        rows.seq_row = d_slot_;
+        rows.wpos = d_wpos_;
+    }
     detail::launch_w8a16(x, hidden, n_, hidden, group_size, segs, nseg, &rows, ws, stream, packed);
     return Result<void>::ok();
 }
@@ -754,7 +758,8 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
 // ======================================================================
 
 PrefillBatch::PrefillBatch(KVCacheManager &mgr, int max_seqs, int num_q_heads)
-    : mgr_(mgr), max_seqs_(max_seqs), num_q_heads_(num_q_heads), meta_(new detail::MetaRing(4)) {}
+    : mgr_(mgr), max_seqs_(max_seqs), num_q_heads_(num_q_heads), meta_(new detail::MetaRing(4)),
+      inl_(new detail::PrefillInline) {}
 
 PrefillBatch::~PrefillBatch() = default;
 
@@ -783,6 +788,7 @@ Result<void> PrefillBatch::prepare(const int *seq_ids, const int *num_tokens, in
     max_keys_ = 0;
     d_work_ = nullptr;
     uploaded_ = false;
+    inline_ok_ = false;
     ids_.clear();
     counts_.clear();
     slots_.clear();
@@ -830,8 +836,14 @@ Result<void> PrefillBatch::prepare(const int *seq_ids, const int *num_tokens, in
     }
     waves_ = detail::prefill_waves(entries.data(), n, cfg.head_dim, num_q_heads_ / cfg.num_heads,
                                    cfg.num_heads, detail::device_cus());
-    detail::plan_prefill(entries.data(), n, cfg.head_dim, num_q_heads_ / cfg.num_heads, waves_, work_);
-    n_items_ = static_cast<int>(work_.size() / detail::kPrefillItemWords);
+    const int group = num_q_heads_ / cfg.num_heads;
+    inline_ok_ = detail::plan_prefill_inline(entries.data(), n, cfg.head_dim, group, waves_, *inl_);
+    if (inline_ok_) {
+        n_items_ = inl_->n_items;
+    } else {
+        detail::plan_prefill(entries.data(), n, cfg.head_dim, group, waves_, work_);
+        n_items_ = static_cast<int>(work_.size() / detail::kPrefillItemWords);
+    }
     slots_ = std::move(slots);
     pos0_.resize(static_cast<size_t>(n));
     for (int i = 0; i < n; ++i) pos0_[static_cast<size_t>(i)] = entries[static_cast<size_t>(i)].p0;
@@ -889,7 +901,7 @@ Result<void> PrefillBatch::launch(int layer_idx, const half *q, const half *new_
          reinterpret_cast<uintptr_t>(new_k) | reinterpret_cast<uintptr_t>(new_v)) & 15u)
         return Result<void>::err("PrefillBatch: q, out, new_k and new_v must be 16-byte aligned");
     if (n_items_ == 0) return Result<void>::ok();
-    upload_device(stream);
+    if (!inline_ok_) upload_device(stream);
     detail::PrefillLaunch p;
     p.q = q;
     p.out = out;
@@ -897,6 +909,7 @@ Result<void> PrefillBatch::launch(int layer_idx, const half *q, const half *new_
     p.q_head_stride = cfg.head_dim;
     p.work = d_work_;
     p.n_items = n_items_;
+    p.inl = inline_ok_ ? inl_.get() : nullptr;
     p.waves = waves_;
     p.max_keys = max_keys_;
     p.new_k = new_k;

@@ -33,6 +33,7 @@ struct WorkList;
 class BlockAllocator;
 struct InlineMeta;
 struct PrefillEntry;
+struct PrefillInline;
 class MetaRing;
 class Workspace;
 } // namespace detail
@@ -270,6 +271,10 @@ class PrefillBatch {
     bool                 uploaded_ = false;
     std::unique_ptr<detail::MetaRing> meta_;
     const int32_t       *d_work_ = nullptr;
+    // The work in the kernel arguments where it fits (then work_ is empty and
+    // nothing is uploaded).
+    std::unique_ptr<detail::PrefillInline> inl_;
+    bool                                   inline_ok_ = false;
 };
 
 } // namespace tiny_llm

@@ -32,7 +32,7 @@ def product(x, w, s, K, gs):
     (128, 18432, 96, 32),    # full tiles, an unpaired last step
     (129, 18304, 160, 128),  # one row over, a partial last scale group
     (257, 9232, 128, 32),    # two groups per chunk, a column tail
-    (320, 7408, 288, 64),    # several row tiles, K % 64 == 32 inside a group
+    (320, 8208, 288, 64),    # several row tiles, K % 64 == 32 inside a group
     (200, 6560, 2080, 512),  # few rows with a long K; groups across chunks and the K halves' boundary
     (2390, 1008, 192, 256),  # more row tiles than a panel, a group longer than K
     (9250, 256, 64, 32),     # one column tile
@@ -86,7 +86,7 @@ def test_w8a16_tile_unaligned_output(tl, orc):
 
 @pytest.mark.parametrize("paged,B,Hkv,D", [
     (False, 130, 2, 64),    # all columns to the split-K kernel
-    (True, 310, 8, 256),    # q to the tile kernel, k and v to the split-K one
+    (True, 650, 8, 128),    # q to the tile kernel, k and v to the split-K one
     (False, 1200, 8, 256),  # all to the tile kernel
     (True, 1200, 8, 256),
 ])

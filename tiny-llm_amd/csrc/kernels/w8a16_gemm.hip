@@ -1471,11 +1471,17 @@ namespace {
 // 600 x 4096 138.6 / 127.1 -> 138.8 / 110.5.  Up to 256 rows the split-K kernel
 // also writes and sums partials when K is 2048 or more: 128 x 11008 40.2 / 39.3
 // -> 32.5 / 27.3, 256 x 8192 54.1 / 53.8 -> 32.9 / 28.8 (but K = 512, 192 x
-// 11008: 10.6 / 11.5 -> 12.1 / 11.2).
+// 11008: 10.6 / 11.5 -> 12.1 / 11.2).  Between 256 and 640 rows and up to 8192
+// columns, where the matrix may be the q part of a decode batch's projection
+// whose k and v parts stay with the split-K kernel, it has to win more than the
+// second launch costs (packed, prepare + project: 350 x (8192 + 2 x 1024) 102 ->
+// 112 us, 580 x (4096 + 2 x 1024) 61 -> 73, both left alone; 600 x (8192 + 2 x
+// 1024) 167 -> 150).
 bool tile_ok(int M, int n, int K) {
     const int64_t outputs = (int64_t)M * n;
     if (M <= 64) return false;
-    return outputs >= (M <= 256 && K >= 2048 ? 5LL << 18 : 9LL << 18);
+    if (M <= 256 && K >= 2048) return outputs >= 5LL << 18;
+    return outputs >= (M > 256 && M <= 640 && n <= 8192 ? 17LL << 18 : 9LL << 18);
 }
 
 // Plan of w8a16_tile_kernel: the tile shape with the least padded work in the

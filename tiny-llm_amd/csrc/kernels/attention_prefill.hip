@@ -383,21 +383,26 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 12
         }
 #pragma unroll
         for (int j = 0; j < NQG; ++j) {
-            float mloc = fmaxf(fmaxf(fmaxf(s[j][0][0], s[j][0][1]), fmaxf(s[j][0][2], s[j][0][3])),
-                               fmaxf(fmaxf(s[j][1][0], s[j][1][1]), fmaxf(s[j][1][2], s[j][1][3])));
-            mloc = fmaxf(mloc, fmaxf(fmaxf(fmaxf(s[j][2][0], s[j][2][1]), fmaxf(s[j][2][2], s[j][2][3])),
-                                     fmaxf(fmaxf(s[j][3][0], s[j][3][1]), fmaxf(s[j][3][2], s[j][3][3]))));
-            mloc = xor_lane_max<16>(mloc);
-            mloc = xor_lane_max<32>(mloc);
+            // The lane's largest score, as a chain of three-operand maxima.
+            float mloc = fmaxf(fmaxf(s[j][0][0], s[j][0][1]), s[j][0][2]);
+            mloc = fmaxf(fmaxf(mloc, s[j][0][3]), s[j][1][0]);
+            mloc = fmaxf(fmaxf(mloc, s[j][1][1]), s[j][1][2]);
+            mloc = fmaxf(fmaxf(mloc, s[j][1][3]), s[j][2][0]);
+            mloc = fmaxf(fmaxf(mloc, s[j][2][1]), s[j][2][2]);
+            mloc = fmaxf(fmaxf(mloc, s[j][2][3]), s[j][3][0]);
+            mloc = fmaxf(fmaxf(mloc, s[j][3][1]), s[j][3][2]);
+            mloc = fmaxf(mloc, s[j][3][3]);
             // Key 0 lies in tile 0 and every query attends it, so the max is
             // finite from the first tile on.  The reference point m_run only
             // moves when the max passes it by more than kLazyMax (log2
             // units): until then p = 2^(x - m_run) <= 2^kLazyMax, exact in
             // fp32 and fp16 range, and the final division by l cancels the
             // shift, so the running sums are rescaled only on such jumps
-            // (once or twice per row instead of on most tiles).
-            const float m_tile = mloc * a.scale_log2;
-            if (__any(m_tile > m_run[j] + kLazyMax)) {
+            // (once or twice per row instead of on most tiles).  Some lane of
+            // the column passes it exactly when the column's max does, so the
+            // max over the column's 4 lanes is taken only then.
+            if (__any(mloc * a.scale_log2 > m_run[j] + kLazyMax)) {
+                const float m_tile = xor_lane_max<32>(xor_lane_max<16>(mloc)) * a.scale_log2;
                 const float m_new = fmaxf(m_run[j], m_tile);
                 const float alpha = __builtin_amdgcn_exp2f(m_run[j] - m_new);
 #pragma unroll

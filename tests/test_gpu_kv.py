@@ -7,7 +7,7 @@ release / re-allocate (stale bytes included) and paged block maps."""
 import numpy as np
 import pytest
 
-from devutil import read_dev, stream, to_dev
+from devutil import read_dev, stream, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -254,3 +254,35 @@ def test_batch_commit_advances_every_sequence(tl):
     assert [g.getSeqLen(s) for s in ids] == [6, 10, 6]
     with pytest.raises(tl.TinyLLMError, match="positive"):
         batch.commit(0)
+
+
+@pytest.mark.parametrize("n,paged,which", [(384, False, "kv"), (385, True, "kv"), (3, True, "v"), (5, False, "k")])
+def test_gather_metadata_forms(tl, n, paged, which):
+    """Gathers whose lengths and rows travel in the kernel arguments (up to 384
+    entries) and through device memory, of both outputs or one."""
+    rng = np.random.default_rng(n)
+    H, D, M, s_max = 2, 32, 48, 41
+    g = tl.KVCacheManager(1, H, D, M, n, **(dict(block_tokens=16, num_blocks=3 * n) if paged else {}))
+    lens = [int(v) for v in rng.integers(1, M, size=n)]
+    k, v = (rng.standard_normal((sum(lens), H * D)).astype(np.float16).view(np.uint16) for _ in range(2))
+    ids = [g.allocateSequence(M)[0] for _ in range(n)]
+    pb = tl.PrefillBatch(g, n, H)
+    pb.prepare(ids, lens, stream())
+    dk, dv = to_dev(k), to_dev(v)
+    pb.append(0, dk.data_ptr(), dv.data_ptr(), stream())
+    pb.commit()
+    order = rng.permutation(n)
+    batch = tl.DecodeBatch(g, n, H)
+    batch.prepare_lengths([ids[i] for i in order], [lens[i] for i in order], stream())
+    outs = {w: to_dev(np.full((n, H, s_max, D), 0x7E00, np.uint16)) for w in which}
+    batch.gather(0, outs["k"].data_ptr() if "k" in which else 0, outs["v"].data_ptr() if "v" in which else 0, s_max,
+                 stream())
+    at = np.concatenate([[0], np.cumsum(lens)])
+    for w, src in (("k", k), ("v", v)):
+        if w not in which:
+            continue
+        got = to_host(outs[w])
+        for b, i in enumerate(order):
+            m = min(lens[i], s_max)
+            rows = src[at[i]:at[i] + m].reshape(m, H, D).transpose(1, 0, 2)
+            assert np.array_equal(got[b, :, :m], rows) and not got[b, :, m:].any()

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 
 namespace tiny_llm {
 namespace detail {
@@ -15,6 +16,7 @@ namespace detail {
 namespace {
 
 constexpr int kCopyThreads = 256;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int64_t row_offset(const KvView &v, int b, int t) {
     const int     row = v.seq_row ? v.seq_row[b] : b;
@@ -91,34 +93,64 @@ __global__ __launch_bounds__(kCopyThreads) void kv_append_ranges_kernel(RangeArg
     *reinterpret_cast<uint4 *>(const_cast<__half *>(a.view.v_base) + dst) = v;
 }
 
+// Attended lengths and cache rows of a gather: in the kernel arguments up to
+// kGatherInline entries, so that the launch needs no metadata copy.
+constexpr int kGatherInline = 384;
+constexpr int kGatherPieces = 2; // 16-byte pieces per thread
 struct GatherArgs {
     KvView         view;
-    const int32_t *lens;
-    int            uniform_len;
+    const int32_t *lens; // device arrays (view.seq_row the rows), or null: the ones below
     int            Hkv;
     int            D;
     int            s_max;
-    const __half  *src;
-    __half        *out;
+    int            n;      // entries
+    const __half  *src[2]; // what grid z counts: n entries of each output, K then V
+    __half        *out[2];
+    int32_t        len[kGatherInline];
+    int32_t        row[kGatherInline];
 };
 
-// grid (ceil(s_max*D/8 / 256), Hkv, n): out[b][g][t][:] from the cache.
+// grid (token blocks, Hkv, outputs * n): out[b][g][t][:] from the cache.  Two
+// pieces per thread, both loads before the stores (one or four: 83 / 76 us where
+// this took 73; kv head fastest in the grid: level to 4% slower).  STREAM:
+// non-temporal stores, for outputs that the L2s (32 MB) cannot hold for their
+// reader: they no longer evict what is still to be read.  (Non-temporal loads
+// too: 68 us where this takes 53.)  Bound by memory: 16 ragged sequences of up
+// to 4096 tokens from 16-token blocks, 8 heads of 128, prepare + gather over
+// three caches in turn 80.7 -> 68.2 us (5.9 TB/s read and written), over one 80.7
+// -> 52.8; 3 sequences of 300 tokens, where the metadata copy and the second
+// launch were most of it, 17.9 -> 10.7.
+template <bool STREAM>
 __global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
-    const int pieces_per_tok = a.D >> 3;
-    const int piece = blockIdx.x * kCopyThreads + threadIdx.x;
-    const int t = piece / pieces_per_tok;
-    if (t >= a.s_max) return;
-    const int e = piece - t * pieces_per_tok;
-    const int g = blockIdx.y;
-    const int b = blockIdx.z;
-    const int len = a.lens ? a.lens[b] : a.uniform_len;
-    uint4     val = make_uint4(0u, 0u, 0u, 0u);
-    if (t < len) {
-        const int64_t off = row_offset(a.view, b, t) + (int64_t)g * a.view.head_stride + e * 8;
-        val = *reinterpret_cast<const uint4 *>(a.src + off);
+    const int z = (int)blockIdx.z, which = z >= a.n, b = z - which * a.n;
+    const int g = (int)blockIdx.y, blk = (int)blockIdx.x;
+    const int ppt = a.D >> 3; // pieces per token
+    const int len = a.lens ? a.lens[b] : a.len[b];
+    const int row = a.lens ? (a.view.seq_row ? a.view.seq_row[b] : b) : a.row[b];
+    const __half *const src = (which ? a.src[1] : a.src[0]) + (int64_t)g * a.view.head_stride;
+    __half *const       out = (which ? a.out[1] : a.out[0]) + ((int64_t)b * a.Hkv + g) * a.s_max * a.D;
+    uint4 val[kGatherPieces];
+#pragma unroll
+    for (int u = 0; u < kGatherPieces; ++u) {
+        const int piece = (blk * kGatherPieces + u) * kCopyThreads + (int)threadIdx.x;
+        const int t = piece / ppt, e = piece - t * ppt;
+        val[u] = make_uint4(0u, 0u, 0u, 0u);
+        if (t < len && t < a.s_max) {
+            const int64_t pb = a.view.block_table
+                                   ? (int64_t)a.view.block_table[(int64_t)row * a.view.bt_stride + (t >> a.view.log2_blk)]
+                                   : row;
+            val[u] = *reinterpret_cast<const uint4 *>(
+                src + pb * a.view.blk_stride + (int64_t)(t & ((1 << a.view.log2_blk) - 1)) * a.view.tok_stride + e * 8);
+        }
     }
-    const int64_t dst = (((int64_t)b * a.Hkv + g) * a.s_max + t) * a.D + e * 8;
-    *reinterpret_cast<uint4 *>(a.out + dst) = val;
+#pragma unroll
+    for (int u = 0; u < kGatherPieces; ++u) {
+        const int piece = (blk * kGatherPieces + u) * kCopyThreads + (int)threadIdx.x;
+        if (piece >= a.s_max * ppt) continue;
+        u32x4 *const dst = reinterpret_cast<u32x4 *>(out + (int64_t)piece * 8);
+        if constexpr (STREAM) __builtin_nontemporal_store(__builtin_bit_cast(u32x4, val[u]), dst);
+        else *dst = __builtin_bit_cast(u32x4, val[u]);
+    }
 }
 
 struct TableArgs {
@@ -210,24 +242,48 @@ void launch_kv_append_ranges(const KvView &view, const int32_t *rows, const int3
     flush();
 }
 
-void launch_kv_gather(const KvView &view, int which, const int32_t *lens, int uniform_len, int n,
-                      int Hkv, int D, int s_max, __half *out, hipStream_t stream) {
-    if (n <= 0 || s_max <= 0 || !out) return;
+bool gather_inline(int n) { return n <= kGatherInline; }
+
+void launch_kv_gather(const KvView &view, const int32_t *lens, const int32_t *host_lens, const int32_t *host_rows, int n,
+                      int Hkv, int D, int s_max, __half *k_out, __half *v_out, hipStream_t stream) {
+    if (n <= 0 || s_max <= 0 || (!k_out && !v_out)) return;
     GatherArgs a;
     a.view = view;
-    a.lens = lens;
-    a.uniform_len = uniform_len;
+    a.lens = gather_inline(n) ? nullptr : lens;
     a.Hkv = Hkv;
     a.D = D;
     a.s_max = s_max;
-    a.src = which ? view.v_base : view.k_base;
-    a.out = out;
-    const long pieces = (long)s_max * (D / 8);
-    dim3       grid((unsigned)((pieces + kCopyThreads - 1) / kCopyThreads), (unsigned)Hkv, (unsigned)n);
-    profile_begin(KernelId::KvGather, stream);
-    hipLaunchKernelGGL(kv_gather_kernel, grid, dim3(kCopyThreads), 0, stream, a);
-    HIP_CHECK(hipGetLastError());
-    profile_end(KernelId::KvGather, stream);
+    a.n = n;
+    if (!a.lens) {
+        std::memcpy(a.len, host_lens, sizeof(int32_t) * (size_t)n);
+        std::memcpy(a.row, host_rows, sizeof(int32_t) * (size_t)n);
+    }
+    const int64_t pieces = (int64_t)s_max * (D / 8), per = (int64_t)kCopyThreads * kGatherPieces;
+    const int64_t blocks = (pieces + per - 1) / per;
+    const int64_t bytes = pieces * 16 * Hkv * n * ((k_out != nullptr) + (v_out != nullptr));
+    auto          go = [&](int outputs) {
+        const dim3 grid((unsigned)blocks, (unsigned)Hkv, (unsigned)(outputs * n));
+        profile_begin(KernelId::KvGather, stream);
+        if (bytes > (32LL << 20))
+            hipLaunchKernelGGL((kv_gather_kernel<true>), grid, dim3(kCopyThreads), 0, stream, a);
+        else
+            hipLaunchKernelGGL((kv_gather_kernel<false>), grid, dim3(kCopyThreads), 0, stream, a);
+        HIP_CHECK(hipGetLastError());
+        profile_end(KernelId::KvGather, stream);
+    };
+    if (k_out && v_out && n <= 65535 / 2) { // one launch for both
+        a.src[0] = view.k_base;
+        a.src[1] = view.v_base;
+        a.out[0] = k_out;
+        a.out[1] = v_out;
+        go(2);
+        return;
+    }
+    for (int which = 0; which < 2; ++which) {
+        a.src[0] = a.src[1] = which ? view.v_base : view.k_base;
+        a.out[0] = a.out[1] = which ? v_out : k_out;
+        if (a.out[0]) go(1);
+    }
 }
 
 } // namespace detail

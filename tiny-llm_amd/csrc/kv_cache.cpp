@@ -689,12 +689,9 @@ Result<void> DecodeBatch::gather(int layer_idx, half *k_out, half *v_out, int s_
         return Result<void>::err("DecodeBatch: Invalid layer_idx: " + std::to_string(layer_idx));
     if (s_max < 0) return Result<void>::err("DecodeBatch: s_max must be >= 0");
     if (n_ == 0 || s_max == 0) return Result<void>::ok();
-    upload_device(stream);
-    const KvView v = mgr_.layerView(layer_idx, d_slot_);
-    if (k_out)
-        detail::launch_kv_gather(v, 0, d_lens_, 0, n_, cfg.num_heads, cfg.head_dim, s_max, k_out, stream);
-    if (v_out)
-        detail::launch_kv_gather(v, 1, d_lens_, 0, n_, cfg.num_heads, cfg.head_dim, s_max, v_out, stream);
+    if (!detail::gather_inline(n_)) upload_device(stream);
+    detail::launch_kv_gather(mgr_.layerView(layer_idx, d_slot_), d_lens_, lens_.data(), slot_.data(), n_, cfg.num_heads,
+                             cfg.head_dim, s_max, k_out, v_out, stream);
     return Result<void>::ok();
 }
 

@@ -17,6 +17,7 @@ namespace {
 
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float    f32x16 __attribute__((ext_vector_type(16)));
 typedef float    f32x32 __attribute__((ext_vector_type(32)));
 
@@ -213,11 +214,13 @@ __global__ __launch_bounds__(256, 3) void attention_weights_kernel(const __half 
 // lanes on consecutive elements.  Bound by memory: 32000 rows of 1000 in 22.4
 // us (5.7 TB/s), of 1001 in 37.7; three passes by 2-byte loads took 70.  One
 // wave per row up to 1024 values (four rows a workgroup, no barrier), beyond
-// it a workgroup, so that a lane holds at most 32 values.
+// it a workgroup, so that a lane holds at most 32 values.  Outputs beyond the L2s'
+// 32 MB are stored non-temporally (nt), which leaves the caches to the inputs
+// still to be read: 32000 x 1000 over four arrays in turn 25-27 -> 21-22 us.
 constexpr float kLog2e = 1.4426950408889634f;
 
 template <int WPR, int NV, bool VEC>
-__global__ __launch_bounds__(256) void softmax_kernel(const __half *in, __half *out, int64_t rows, int S) {
+__global__ __launch_bounds__(256) void softmax_kernel(const __half *in, __half *out, int64_t rows, int S, bool nt) {
     constexpr int T = 64 * WPR; // lanes of a row
     __shared__ float red[8];
     const int     lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -273,9 +276,13 @@ __global__ __launch_bounds__(256) void softmax_kernel(const __half *in, __half *
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = __builtin_bit_cast(uint16_t, (_Float16)materialize(e[v][j] * inv));
         if constexpr (VEC) {
-            uint4 p;
+            u32x4 p;
             __builtin_memcpy(&p, o, 16);
-            if (at(v, 0) < S) *reinterpret_cast<uint4 *>(y + at(v, 0)) = p;
+            u32x4 *const dst = reinterpret_cast<u32x4 *>(y + at(v, 0));
+            if (at(v, 0) < S) {
+                if (nt) __builtin_nontemporal_store(p, dst);
+                else *dst = p;
+            }
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j)
@@ -311,12 +318,13 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 template <bool VEC>
 void launch_softmax_v(const __half *in, __half *out, int rows, int S, hipStream_t stream) {
+    const bool nt = (int64_t)rows * S * 2 > (32LL << 20); // more than the L2s hold for the reader
     const dim3 per4((unsigned)(((int64_t)rows + 3) / 4)), per1((unsigned)rows), block(256);
-    if (S <= 512) hipLaunchKernelGGL((softmax_kernel<1, 1, VEC>), per4, block, 0, stream, in, out, (int64_t)rows, S);
-    else if (S <= 1024) hipLaunchKernelGGL((softmax_kernel<1, 2, VEC>), per4, block, 0, stream, in, out, (int64_t)rows, S);
-    else if (S <= 2048) hipLaunchKernelGGL((softmax_kernel<4, 1, VEC>), per1, block, 0, stream, in, out, (int64_t)rows, S);
-    else if (S <= 4096) hipLaunchKernelGGL((softmax_kernel<4, 2, VEC>), per1, block, 0, stream, in, out, (int64_t)rows, S);
-    else if (S <= 8192) hipLaunchKernelGGL((softmax_kernel<4, 4, VEC>), per1, block, 0, stream, in, out, (int64_t)rows, S);
+    if (S <= 512) hipLaunchKernelGGL((softmax_kernel<1, 1, VEC>), per4, block, 0, stream, in, out, (int64_t)rows, S, nt);
+    else if (S <= 1024) hipLaunchKernelGGL((softmax_kernel<1, 2, VEC>), per4, block, 0, stream, in, out, (int64_t)rows, S, nt);
+    else if (S <= 2048) hipLaunchKernelGGL((softmax_kernel<4, 1, VEC>), per1, block, 0, stream, in, out, (int64_t)rows, S, nt);
+    else if (S <= 4096) hipLaunchKernelGGL((softmax_kernel<4, 2, VEC>), per1, block, 0, stream, in, out, (int64_t)rows, S, nt);
+    else if (S <= 8192) hipLaunchKernelGGL((softmax_kernel<4, 4, VEC>), per1, block, 0, stream, in, out, (int64_t)rows, S, nt);
     else hipLaunchKernelGGL(softmax_long_kernel, per1, block, 0, stream, in, out, S);
 }
 

@@ -475,7 +475,9 @@ struct DecArgs {
     // Cache row and write position of each entry: in the arguments, because a
     // host-to-device copy in front of the launch takes a third as long as the
     // kernel (prepare + project of a Llama-3-8B layer: 64 entries 17.4 -> 11.0
-    // us, 4 entries 13.8 -> 9.4).
+    // us, 4 entries 13.8 -> 9.4).  The larger arguments cost 0.5 us where several
+    // calls share one prepare (9.4 -> 9.9 a call), whichever memory the rows are
+    // then read from and wherever in the kernel.
     int32_t       row[kDecRows];
     int32_t       wpos[kDecRows];
 };

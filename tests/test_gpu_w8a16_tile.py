@@ -70,6 +70,42 @@ def test_w8a16_tile_scales(tl, orc):
     assert np.array_equal(np.where(got == 0x8000, 0, got), got_p)
 
 
+def test_w8a16_tile_infinite_scales(tl, orc):
+    """Infinite and NaN scales: what folding each group's product gives, +-inf
+    by the product's sign (two infinite groups in a row, or one before a zero
+    scale, included), NaN where it is zero."""
+    M, N, K, gs = 2047, 4080, 512, 64
+    rng = np.random.default_rng(9)
+    x, w, s = operands(orc, rng, M, N, K, gs)
+    f = s.view(np.float16).reshape(K // gs, N)
+    inf = np.inf
+    for col, groups in {20: {2: inf}, 21: {2: inf, 3: inf}, 22: {2: inf, 3: 0}, 23: {0: inf}, 24: {7: inf},
+                        25: {1: inf, 3: inf}, 26: {2: -inf}, 27: {2: inf, 3: -inf}, 28: {2: np.nan}, 29: {2: inf},
+                        30: {2: 0, 3: inf}, 31: {1: inf, 6: inf}}.items():
+        for g, v in groups.items():
+            f[g, col] = v
+    w[128:192, 29] = 0
+    cols = np.arange(20, 32)
+    # K halves of four groups each: (half, group, row, column)
+    p = np.einsum("mgk,gkc->gmc", x.view(np.float16).astype(np.float64).reshape(M, 8, 64),
+                  w[:, cols].astype(np.float64).reshape(8, 64, -1)).reshape(2, 4, M, -1)
+    with np.errstate(invalid="ignore"):
+        ref = (p * f[:, None, cols].astype(np.float64).reshape(2, 4, 1, -1)).sum(axis=1).sum(axis=0)
+    got, got_p = both(tl, to_dev(x), w, to_dev(s), M, N, K, gs)
+    g = got.view(np.float16).astype(np.float64)
+    # (opposite infinities within a half: not a number in the fold, not finite here)
+    same = (g[:, cols] == ref) | (np.isnan(g[:, cols]) & np.isnan(ref))
+    clash = np.isin(cols, (21, 25, 27)) & np.isnan(ref) & np.isinf(g[:, cols])
+    assert np.all(same | clash)
+    assert np.isinf(ref[:, [0, 2, 3, 4, 6, 10]]).all() and np.isinf(ref[:, 1]).sum() > M // 4
+    other = np.ones(N, bool)
+    other[cols] = False
+    sc = np.repeat(f[:, other].astype(np.float64), gs, axis=0)
+    assert rows_close(got[:, other], x.view(np.float16).astype(np.float64) @ (w[:, other] * sc)) <= TOL
+    h = got_p.view(np.float16).astype(np.float64)
+    assert np.all((g == h) | (np.isnan(g) & np.isnan(h)))
+
+
 def test_w8a16_tile_unaligned_output(tl, orc):
     """An output base two bytes past a 16-byte boundary: element stores, and
     nothing outside the matrix is written."""

@@ -890,6 +890,9 @@ __device__ __forceinline__ void epilogue8(const GemmArgs &a, int si, int m, int 
 // output instead of two, which is what lets a wave hold 128 x 64 outputs.  A
 // zero scale keeps the last nonzero one and zeroes its columns' weights
 // instead.  At the end T * s of the two K halves are added through LDS.
+// Infinite and NaN scales give what folding each group's product would: +-inf
+// by the sign of the product, NaN where it is zero (only of two infinite groups
+// of opposite signs in one K half the first wins, where a fold gives NaN).
 //
 // The order of an output's sum depends on K and the group size only, never on
 // the tile shape, the columns or the other segments.
@@ -1099,17 +1102,38 @@ __global__ __launch_bounds__(512, 2) void w8a16_tile_kernel(TileArgs ta) {
     }
     // A scale group begins: T, still 0 before the first, goes over to its units.
     auto new_group = [&](const uint16_t(&sc)[CB]) __attribute__((always_inline)) {
+        float se[CB], ratio[CB];
+        float most = 0.0f;
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
             const float sn = h2f(__builtin_bit_cast(__half, sc[cb]));
             zero[cb] = sn == 0.0f;
-            const float se = zero[cb] ? s_cur[cb] : sn;
-            const float ratio = s_cur[cb] / se;
+            se[cb] = zero[cb] ? s_cur[cb] : sn;
+            ratio[cb] = s_cur[cb] / se[cb];
+            most = fmaxf(most, fabsf(se[cb]));
+        }
+        if (__builtin_expect(__any(__builtin_isinf(most)), 0)) {
+            // Units of an infinite scale: the sum so far is an infinity, NaN or, beside it, nothing.
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                const bool ci = __builtin_isinf(se[cb]);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float v = acc[rb][cb][i] * s_cur[cb];
+                        acc[rb][cb][i] = !ci ? acc[rb][cb][i] : __builtin_isfinite(v) ? 0.0f : v;
+                    }
+                ratio[cb] = ci ? copysignf(1.0f, se[cb]) : ratio[cb];
+            }
+        }
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[rb][cb][i] *= ratio;
-            s_cur[cb] = se;
+                for (int i = 0; i < 4; ++i) acc[rb][cb][i] *= ratio[cb];
+            s_cur[cb] = se[cb];
         }
     };
     auto multiply = [&](const f16x8(&xa)[RB], uint2 raw, int cb) __attribute__((always_inline)) {

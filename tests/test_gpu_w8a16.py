@@ -6,6 +6,7 @@ MFMA path; bit-exact fp16 for the reference-order kernel; bit-exact cache
 bytes between the fused projection and w8a16_matmul + appendKV(n=1)."""
 import numpy as np
 import pytest
+import torch
 
 from devutil import empty_dev, read_dev, rel_err, stream, to_dev, to_dev_raw, to_host
 
@@ -242,6 +243,97 @@ def _cache(tl, orc, rng, L, Hkv, D, M, lens, paged):
         o.advance(sid, S)
         ids.append(sid)
     return g, o, ids, keep
+
+
+def _layer_projections(tl, orc, rng, L, Hkv, G, D, hidden, gs):
+    """Per-layer K and V weights on the device, and calls that project a batch
+    fused and as separate products plus append."""
+    row = Hkv * D
+    ws = [[operands(orc, rng, 1, row, hidden, gs)[1:] for _ in range(2)] for _ in range(L)]
+    dev = [[(to_dev_raw(w), to_dev(s)) for w, s in kv] for kv in ws]
+
+    def fused(batch, layer, dx, st):
+        (wk, sk), (wv, sv) = dev[layer]
+        batch.project(layer, dx.data_ptr(), hidden, gs, wk.data_ptr(), sk.data_ptr(), wv.data_ptr(), sv.data_ptr(),
+                      stream=st)
+
+    def separate(batch, layer, dx, st):
+        out = [empty_dev((dx.shape[0], row)) for _ in range(2)]
+        for (w, s), o in zip(dev[layer], out):
+            tl.w8a16_matmul(dx.data_ptr(), w.data_ptr(), s.data_ptr(), o.data_ptr(), dx.shape[0], row, hidden, gs, st)
+        batch.append(layer, 1, out[0].data_ptr(), out[1].data_ptr(), st)
+        return out
+    return fused, separate
+
+
+@pytest.mark.parametrize("paged", [False, True])
+def test_project_every_layer_of_a_step(tl, orc, paged):
+    """A step's projections after its first read the rows that the first one
+    left on the device: every layer's cache bytes are those of the separate
+    products, over steps of different order and size, after an append of the
+    same step (rows already on the device), and on two streams."""
+    L, Hkv, G, D, hidden, gs, n = 5, 2, 4, 64, 256, 64, 40
+    lens = [int(v) for v in np.random.default_rng(3).integers(1, 60, size=n)]
+    g, _, ids, keep = _cache(tl, orc, np.random.default_rng(12), L, Hkv, D, 96, lens, paged)
+    g2, _, ids2, keep2 = _cache(tl, orc, np.random.default_rng(12), L, Hkv, D, 96, lens, paged)
+    rng = np.random.default_rng(13)
+    fused, separate = _layer_projections(tl, orc, rng, L, Hkv, G, D, hidden, gs)
+    a, b = tl.DecodeBatch(g, n, Hkv * G), tl.DecodeBatch(g2, n, Hkv * G)
+    other = torch.cuda.Stream()
+    for step in range(7):  # more steps than device buffers
+        order = rng.permutation(n)[:1 + 13 * step % n]
+        dx = to_dev(orc.f2h(rng.standard_normal((len(order), hidden)).astype(np.float32)))
+        a.prepare([ids[i] for i in order], stream())
+        b.prepare([ids2[i] for i in order], stream())
+        kept = []
+        for layer in range(L):
+            kept.append(separate(b, layer, dx, stream()))
+            if step == 3 and layer == 2:
+                a.append(4, 1, kept[0][0].data_ptr(), kept[0][1].data_ptr(), stream())
+            if step == 5 and layer in (1, 3):
+                torch.cuda.synchronize()
+                fused(a, layer, dx, other.cuda_stream)
+                torch.cuda.synchronize()
+            else:
+                fused(a, layer, dx, stream())
+        for m, batch in ((g, a), (g2, b)):
+            batch.commit(1)
+        torch.cuda.synchronize()
+    elems = g.slot_bytes() // 2 * (n + 1)
+    assert np.array_equal(read_dev(g.pool(), elems), read_dev(g2.pool(), elems))
+
+
+def test_project_replays_under_hip_graph_capture(tl, orc):
+    """Projections of every layer in a graph, with eager steps between the
+    replays: each replay leaves the bytes of the step it was captured from."""
+    L, Hkv, G, D, hidden, gs, n = 3, 2, 4, 64, 256, 64, 9
+    lens = list(range(1, n + 1))
+    g, _, ids, keep = _cache(tl, orc, np.random.default_rng(14), L, Hkv, D, 96, lens, False)
+    rng = np.random.default_rng(15)
+    fused, separate = _layer_projections(tl, orc, rng, L, Hkv, G, D, hidden, gs)
+    dx = to_dev(orc.f2h(rng.standard_normal((n, hidden)).astype(np.float32)))
+    batch = tl.DecodeBatch(g, n, Hkv * G)
+    batch.prepare(ids, stream())
+    for layer in range(L):
+        fused(batch, layer, dx, stream())
+    elems = g.slot_bytes() // 2 * (n + 1)
+    want = read_dev(g.pool(), elems)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for layer in range(L):
+            fused(batch, layer, dx, stream())
+    torch.cuda.synchronize()
+    noise = to_dev(orc.f2h(rng.standard_normal((n, hidden)).astype(np.float32)))
+    for rep in range(3):
+        for _ in range(3):  # other rows through every device buffer, over the same positions
+            order = rng.permutation(n)
+            batch.prepare([ids[i] for i in order], stream())
+            for layer in range(L):
+                fused(batch, layer, noise, stream())
+        assert not np.array_equal(read_dev(g.pool(), elems), want)
+        graph.replay()
+        assert np.array_equal(read_dev(g.pool(), elems), want), rep
+    del graph
 
 
 @pytest.mark.parametrize("packed", [False, True])

@@ -40,7 +40,8 @@ def kernels(obj, tmp_path):
         if name.endswith(".kd"):
             continue
         out[name] = {k: int(re.search(rf"\.{k}:\s+(\d+)", blk).group(1))
-                     for k in ("private_segment_fixed_size", "vgpr_spill_count", "vgpr_count")}
+                     for k in ("private_segment_fixed_size", "vgpr_spill_count", "vgpr_count",
+                               "kernarg_segment_size")}
     assert out, "no kernels found"
     return out
 
@@ -91,3 +92,17 @@ def test_prefill_kernels_spill_nothing(tmp_path):
     assert len(pf) == 3 * 4 * 2 * 2 + 4 * 2, sorted(pf)
     bad = {n: r for n, r in pf.items() if r["vgpr_spill_count"] or r["private_segment_fixed_size"]}
     assert not bad, bad
+
+
+def test_w8a16_dec_arguments(tmp_path):
+    """Cache rows travel in the arguments of a step's first projection only:
+    every other product of w8a16_dec_kernel, and the further projections of the
+    step, keep arguments of a few cache lines (512 bytes more cost a launch
+    2-3%).  Neither form uses scratch memory."""
+    ks = kernels("w8a16_gemm.o", tmp_path)
+    dec = {n: r for n, r in ks.items() if "w8a16_dec_kernel" in n}
+    rows = {n: r for n, r in ks.items() if "w8a16_dec_rows_kernel" in n}
+    assert len(dec) == len(rows) == 16
+    assert max(r["kernarg_segment_size"] for r in dec.values()) <= 384
+    for name, r in rows.items():
+        assert r["private_segment_fixed_size"] == 0 and r["vgpr_spill_count"] == 0, (name, r)

@@ -24,21 +24,29 @@ struct W8A16Seg {
     const __half *res = nullptr; // residual: same layout as out (may alias out)
 };
 
+// Rows that w8a16_dec_kernel takes at most.
+constexpr int kDecRows = 64;
+
 // Destination rows of the cache epilogue: entry m's token row at write
 // position wpos[m] of cache row seq_row[m] (block-table addressing when
 // block_table is set; see KvView).
 struct CacheRows {
     const int32_t *seq_row = nullptr;
     const int32_t *wpos = nullptr;
-    // The same arrays in host memory: enough where w8a16_takes_dec says so (that
-    // kernel has them in its arguments), and seq_row / wpos may then be null.
-    const int32_t *host_row = nullptr;
-    const int32_t *host_wpos = nullptr;
     const int32_t *block_table = nullptr;
     int            bt_stride = 0;
     int            log2_blk = 30;
     int64_t        blk_stride = 0;
     int64_t        tok_stride = 0;
+};
+
+struct CacheDest : CacheRows {
+    // With seq_row null, where w8a16_takes_dec says so: the same arrays in host
+    // memory.  The launch has them in its arguments, and leaves them in `store`
+    // ([rows | positions], device memory, may be null) for further launches.
+    const int32_t *host_row = nullptr;
+    const int32_t *host_wpos = nullptr;
+    int32_t       *store = nullptr;
 };
 
 // True when the MFMA path covers the shape (K % 32 == 0, gs a power of two in
@@ -63,7 +71,7 @@ bool w8a16_takes_dec(const __half *x, int64_t ldx, int M, int K, int gs, const W
 // packed: every segment's w is in the layout of launch_w8a16_pack (MFMA
 // path only; shapes it does not cover are rejected).
 void launch_w8a16(const __half *x, int64_t ldx, int M, int K, int gs, const W8A16Seg *segs, int nseg,
-                  const CacheRows *cache, float *workspace, hipStream_t stream, bool packed = false);
+                  const CacheDest *cache, float *workspace, hipStream_t stream, bool packed = false);
 
 // W [K][N] int8 -> the MFMA-fragment layout (K % 32 == 0, N % 16 == 0; K*N
 // bytes): fragment (column block nb, k step ks) holds, for lane l, rows

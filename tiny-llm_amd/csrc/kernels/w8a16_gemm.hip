@@ -54,6 +54,7 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 namespace tiny_llm {
 namespace detail {
@@ -454,7 +455,6 @@ __global__ __launch_bounds__(256, ACC ? 2 : 3) void w8a16_sk_kernel(GemmArgs a) 
 // on the column tiling or the segments sharing the launch, so the fused
 // projection's cache bytes equal the unfused product's, and both weight
 // layouts give the same bits.
-constexpr int kDecRows = 64;   // the kernel's M limit
 constexpr int kDecMaxK = 4096; // and K limit (a multiple of 128): 4 chunks per wave
 constexpr int kDecHalf = 32;   // rows per workgroup
 constexpr int kDecWaves = 8;
@@ -471,15 +471,21 @@ struct DecArgs {
     int           blocks; // 16-column blocks over all segments
     W8A16Seg      seg[kMaxSegs];
     int           col0[kMaxSegs + 1];
-    CacheRows     cache; // block table and strides (rows and positions below)
-    // Cache row and write position of each entry: in the arguments, because a
-    // host-to-device copy in front of the launch takes a third as long as the
-    // kernel (prepare + project of a Llama-3-8B layer: 64 entries 17.4 -> 11.0
-    // us, 4 entries 13.8 -> 9.4).  The larger arguments cost 0.5 us where several
-    // calls share one prepare (9.4 -> 9.9 a call), whichever memory the rows are
-    // then read from and wherever in the kernel.
-    int32_t       row[kDecRows];
-    int32_t       wpos[kDecRows];
+    CacheRows     cache;
+};
+
+// The first projection of a prepared step: cache row and write position of each
+// entry in the arguments, because a host-to-device copy in front of the launch
+// takes a third as long as the kernel (prepare + project of a Llama-3-8B layer:
+// 64 entries 17.4 -> 11.0 us, 4 entries 13.8 -> 9.4).  Arguments larger by 512
+// bytes cost a launch 0.2 us, so the kernel leaves the rows in device memory for
+// the step's further projections, and those and every product without cache
+// rows keep the small ones (prepare + 32 projections
+// of 64 entries: 335 us with the copy, 341 with the rows in every launch, 332 so).
+struct DecRowArgs : DecArgs {
+    int32_t  row[kDecRows];
+    int32_t  wpos[kDecRows];
+    int32_t *store; // [M rows | M positions], or null
 };
 
 // Field f of segment si (uniform), with static indices only.
@@ -506,8 +512,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t dec_rsrc(const void *p, uint32
 
 // FS: k steps per scale fold (gs / 32, at most 4 = one chunk).  CB: column
 // blocks per tile.  PACKED: W in the launch_w8a16_pack layout.
-template <int FS, int CB, bool PACKED>
-__global__ __launch_bounds__(512, 1) void w8a16_dec_kernel(DecArgs a) {
+// Args by value: through a reference they are copied to scratch memory.
+template <int FS, int CB, bool PACKED, class Args>
+__device__ __forceinline__ void dec_body(Args a) {
+    constexpr bool ROWS = std::is_same_v<Args, DecRowArgs>;
     static_assert(FS == 1 || FS == 2 || FS == 4, "fold");
     static_assert(CB >= 1 && CB <= 4, "column blocks");
     constexpr int NF = 4 / FS;                                  // folds per chunk
@@ -583,8 +591,13 @@ __global__ __launch_bounds__(512, 1) void w8a16_dec_kernel(DecArgs a) {
     if (eact && ekind == kEpiCache) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            erow[i] = (uint32_t)a.row[em[i]];
-            epos[i] = (uint32_t)a.wpos[em[i]];
+            if constexpr (ROWS) {
+                erow[i] = (uint32_t)a.row[em[i]];
+                epos[i] = (uint32_t)a.wpos[em[i]];
+            } else {
+                erow[i] = (uint32_t)a.cache.seq_row[em[i]];
+                epos[i] = (uint32_t)a.cache.wpos[em[i]];
+            }
         }
     } else if (eact && ekind == kEpiResidual) {
         const __half *res = TL_DEC_SEG(a, esi, res);
@@ -828,6 +841,23 @@ __global__ __launch_bounds__(512, 1) void w8a16_dec_kernel(DecArgs a) {
         } else {
             out[(int64_t)m * ld + en] = o;
         }
+    }
+}
+
+template <int FS, int CB, bool PACKED>
+__global__ __launch_bounds__(512, 1) void w8a16_dec_kernel(DecArgs a) {
+    dec_body<FS, CB, PACKED>(a);
+}
+
+template <int FS, int CB, bool PACKED>
+__global__ __launch_bounds__(512, 1) void w8a16_dec_rows_kernel(DecRowArgs a) {
+    dec_body<FS, CB, PACKED>(a);
+    // At the end, by a wave without outputs of its own: in front of the weight
+    // stream the wait for these loads cost 0.4 us.
+    const int m = (int)threadIdx.x - 512 + kDecRows;
+    if (a.store && blockIdx.x == 0 && m >= 0 && m < a.M) {
+        a.store[m] = a.row[m];
+        a.store[a.M + m] = a.wpos[m];
     }
 }
 
@@ -1594,8 +1624,8 @@ size_t w8a16_workspace_floats(int M, int K, int gs, const W8A16Seg *segs, int ns
 
 namespace {
 // The decode-sized launch: g's x, shape, segments and cache rows are set.
-void launch_dec(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
-    DecArgs a;
+void launch_dec(const GemmArgs &g, const CacheDest *dest, int gs, hipStream_t stream, bool packed) {
+    DecRowArgs a;
     std::memset(&a, 0, sizeof(a));
     a.x = g.x;
     a.ldx = g.ldx;
@@ -1604,17 +1634,21 @@ void launch_dec(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
     a.gs = gs;
     a.log2_gs = __builtin_ctz((unsigned)gs); // a power of two (w8a16_mfma_ok)
     a.nseg = g.nseg;
-    for (int i = 0; i < g.nseg; ++i) a.seg[i] = g.seg[i];
+    bool to_cache = false;
+    for (int i = 0; i < g.nseg; ++i) {
+        a.seg[i] = g.seg[i];
+        to_cache |= g.seg[i].kind == kEpiCache;
+    }
     for (int i = 0; i <= g.nseg; ++i) a.col0[i] = g.col0[i];
     a.cache = g.cache;
-    for (int i = 0; i < g.nseg; ++i)
-        if (g.seg[i].kind == kEpiCache) {
-            if (!g.cache.host_row || !g.cache.host_wpos)
-                throw std::invalid_argument("w8a16: cache epilogue without host cache rows");
-            std::memcpy(a.row, g.cache.host_row, sizeof(int32_t) * (size_t)g.M);
-            std::memcpy(a.wpos, g.cache.host_wpos, sizeof(int32_t) * (size_t)g.M);
-            break;
-        }
+    const bool rows = to_cache && !g.cache.seq_row;
+    if (rows) {
+        if (!dest->host_row || !dest->host_wpos)
+            throw std::invalid_argument("w8a16: cache epilogue without cache rows");
+        std::memcpy(a.row, dest->host_row, sizeof(int32_t) * (size_t)g.M);
+        std::memcpy(a.wpos, dest->host_wpos, sizeof(int32_t) * (size_t)g.M);
+        a.store = dest->store;
+    }
     const DecPlan p = dec_plan(g.M, gs, g.seg, g.nseg);
     a.tiles = p.tiles;
     a.tpx = (p.tiles + 7) / 8;
@@ -1623,12 +1657,18 @@ void launch_dec(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
     const unsigned grid = (unsigned)(8 * a.tpx * p.halves);
     const int      fs = gs >= 128 ? 4 : gs / 32;
     profile_begin(KernelId::W8A16, stream);
-#define TL_W8_DEC(FS, CB)                                                                                  \
-    do {                                                                                                   \
-        if (packed)                                                                                        \
-            hipLaunchKernelGGL((w8a16_dec_kernel<FS, CB, true>), dim3(grid), dim3(512), 0, stream, a);     \
-        else                                                                                               \
-            hipLaunchKernelGGL((w8a16_dec_kernel<FS, CB, false>), dim3(grid), dim3(512), 0, stream, a);    \
+    const DecArgs &small = a;
+#define TL_W8_DEC_P(FS, CB, P)                                                                                \
+    do {                                                                                                      \
+        if (rows)                                                                                             \
+            hipLaunchKernelGGL((w8a16_dec_rows_kernel<FS, CB, P>), dim3(grid), dim3(512), 0, stream, a);      \
+        else                                                                                                  \
+            hipLaunchKernelGGL((w8a16_dec_kernel<FS, CB, P>), dim3(grid), dim3(512), 0, stream, small);       \
+    } while (0)
+#define TL_W8_DEC(FS, CB)                      \
+    do {                                       \
+        if (packed) TL_W8_DEC_P(FS, CB, true); \
+        else TL_W8_DEC_P(FS, CB, false);       \
     } while (0)
     if (fs == 4) {
         switch (p.cb) {
@@ -1645,6 +1685,7 @@ void launch_dec(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
         else TL_W8_DEC(1, 2);
     }
 #undef TL_W8_DEC
+#undef TL_W8_DEC_P
     HIP_CHECK(hipGetLastError());
     profile_end(KernelId::W8A16, stream);
 }
@@ -1665,7 +1706,7 @@ bool w8a16_takes_dec(const __half *x, int64_t ldx, int M, int K, int gs, const W
 }
 
 void launch_w8a16(const __half *x, int64_t ldx, int M, int K, int gs, const W8A16Seg *segs, int nseg,
-                  const CacheRows *cache, float *workspace, hipStream_t stream, bool packed) {
+                  const CacheDest *cache, float *workspace, hipStream_t stream, bool packed) {
     if (nseg < 1 || nseg > kMaxSegs) throw std::invalid_argument("w8a16: 1..3 weight segments");
     GemmArgs a;
     std::memset(&a, 0, sizeof(a));
@@ -1702,7 +1743,7 @@ void launch_w8a16(const __half *x, int64_t ldx, int M, int K, int gs, const W8A1
         return;
     }
     if (dec_ok(M, K, segs, nseg)) {
-        launch_dec(a, gs, stream, packed);
+        launch_dec(a, cache, gs, stream, packed);
         return;
     }
     // Large segments to the tile kernel, the others to the split-K one.

@@ -474,7 +474,7 @@ DecodeBatch::DecodeBatch(KVCacheManager &mgr, int max_seqs, int num_q_heads)
     : mgr_(mgr), max_seqs_(max_seqs), num_q_heads_(num_q_heads), meta_(new detail::MetaRing(4)),
       work_(new detail::Workspace()), gemm_work_(new detail::Workspace()),
       plan_(new detail::WorkList()),
-      inl_(new detail::InlineMeta()) {}
+      inl_(new detail::InlineMeta()), rows_(new detail::DeviceRing()) {}
 
 DecodeBatch::~DecodeBatch() = default;
 
@@ -500,6 +500,7 @@ Result<std::unique_ptr<DecodeBatch>> DecodeBatch::create(KVCacheManager &mgr, in
     const size_t n = static_cast<size_t>(max_seqs);
     const size_t words = 4 * n + 1 + 2 * (n + slots);
     batch->meta_->reserve(std::min<size_t>(words * 4, size_t(4) << 20));
+    batch->rows_->reserve(2 * sizeof(int32_t) * std::min<size_t>(n, detail::kDecRows));
     return R::ok(std::move(batch));
 }
 
@@ -512,6 +513,7 @@ Result<void> DecodeBatch::upload(const int *seq_ids, const int *attended, int n,
     // A failed prepare leaves an empty batch.
     n_ = 0;
     appendable_ = false;
+    d_rows_ = nullptr;
     ids_.clear();
     const KVCacheConfig &cfg = mgr_.getConfig();
     std::vector<char>    taken(static_cast<size_t>(cfg.max_batch_size), 0);
@@ -712,7 +714,7 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
         return Result<void>::err("DecodeBatch: wq, sq and q_out must be all set or all null");
     if (n_ == 0) return Result<void>::ok();
     const KvView v = mgr_.layerView(layer_idx, nullptr);
-    detail::CacheRows rows;
+    detail::CacheDest rows;
     rows.host_row = slot_.data();
     rows.host_wpos = wpos_.data();
     rows.block_table = v.block_table;
@@ -741,12 +743,25 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
     if (packed && !detail::w8a16_mfma_ok(hidden, group_size, segs, nseg))
         return Result<void>::err("DecodeBatch: packed weights need hidden % 32 == 0 and group_size "
                                  "in {32, 64, 128, 256, 512}");
-    if (!detail::w8a16_takes_dec(x, hidden, n_, hidden, group_size, segs, nseg, packed)) {
-        upload_device(stream); // the other kernels read the rows from device memory
+    int32_t *store = nullptr;
+    if (uploaded_ || !detail::w8a16_takes_dec(x, hidden, n_, hidden, group_size, segs, nseg, packed)) {
+        upload_device(stream); // (the other kernels read the rows from device memory)
         rows.seq_row = d_slot_;
         rows.wpos = d_wpos_;
+    } else if (detail::stream_capturing(stream)) {
+        // A captured launch keeps its rows in its arguments: replays then depend
+        // on nothing that later steps rewrite.
+    } else if (d_rows_ && rows_stream_ == stream) {
+        rows.seq_row = d_rows_;
+        rows.wpos = d_rows_ + n_;
+    } else {
+        store = rows.store = rows_->next();
     }
     detail::launch_w8a16(x, hidden, n_, hidden, group_size, segs, nseg, &rows, ws, stream, packed);
+    if (store) {
+        d_rows_ = store;
+        rows_stream_ = stream;
+    }
     return Result<void>::ok();
 }
 

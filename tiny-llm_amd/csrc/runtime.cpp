@@ -84,6 +84,31 @@ int device_cus() {
     return v;
 }
 
+bool stream_capturing(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true; // (the default stream beside a capture: the launch itself will report it)
+}
+
+// -------------------------------------------------------------- DeviceRing
+DeviceRing::~DeviceRing() {
+    if (base_) {
+        (void)hipDeviceSynchronize(); // kernels queued on callers' streams may still read it
+        (void)hipFree(base_);
+    }
+}
+
+void DeviceRing::reserve(size_t bytes) {
+    bytes_ = (bytes + 255) & ~size_t(255);
+    HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&base_), kSlots * bytes_));
+}
+
+int32_t *DeviceRing::next() {
+    cur_ = (cur_ + 1) % kSlots;
+    return reinterpret_cast<int32_t *>(base_ + static_cast<size_t>(cur_) * bytes_);
+}
+
 // ---------------------------------------------------------------- MetaRing
 MetaRing::MetaRing(int slots) : slots_(static_cast<size_t>(slots)) {}
 

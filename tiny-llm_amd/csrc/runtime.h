@@ -5,6 +5,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstddef>
+#include <cstdint>
 #include <mutex>
 #include <vector>
 
@@ -49,6 +50,29 @@ class MetaRing {
     int                 cur_ = -1;
     size_t              bytes_ = 0;
 };
+
+// Ring of equal device buffers that kernels fill: what the first launch of a
+// step brings in its arguments, kept for the step's further launches.  One
+// allocation, made by reserve(); a buffer is written again after three others,
+// in stream order behind the kernels that read it.
+class DeviceRing {
+  public:
+    DeviceRing() = default;
+    ~DeviceRing();
+    DeviceRing(const DeviceRing &) = delete;
+    DeviceRing &operator=(const DeviceRing &) = delete;
+    void     reserve(size_t bytes);
+    int32_t *next();
+
+  private:
+    static constexpr int kSlots = 4;
+    char  *base_ = nullptr;
+    size_t bytes_ = 0;
+    int    cur_ = 0;
+};
+
+// Whether work queued on the stream is being captured into a graph.
+bool stream_capturing(hipStream_t stream);
 
 // Grow-only device buffer (split-K partials).
 class Workspace {

@@ -35,6 +35,7 @@ struct InlineMeta;
 struct PrefillEntry;
 struct PrefillInline;
 class MetaRing;
+class DeviceRing;
 class Workspace;
 } // namespace detail
 
@@ -213,6 +214,11 @@ class DecodeBatch {
     bool                               uploaded_ = false;  // device copy of this prepare made
     const int32_t  *d_lens_ = nullptr, *d_wpos_ = nullptr, *d_slot_ = nullptr;
     const int32_t  *d_part_base_ = nullptr, *d_work_ = nullptr;
+    // Rows and positions that this prepare's first projection left in device
+    // memory, on rows_stream_, for the next ones (null: none has yet).
+    std::unique_ptr<detail::DeviceRing> rows_;
+    const int32_t                      *d_rows_ = nullptr;
+    hipStream_t                         rows_stream_ = nullptr;
 };
 
 // A prefill step over n sequences of one manager: sequence i brings

@@ -471,10 +471,11 @@ KvView KVCacheManager::layerView(int layer_idx, const int32_t *seq_row_dev) cons
 // ======================================================================
 
 DecodeBatch::DecodeBatch(KVCacheManager &mgr, int max_seqs, int num_q_heads)
-    : mgr_(mgr), max_seqs_(max_seqs), num_q_heads_(num_q_heads), meta_(new detail::MetaRing(4)),
+    : mgr_(mgr), max_seqs_(max_seqs), num_q_heads_(num_q_heads),
+      meta_(new detail::MetaRing(4, 2 * sizeof(int32_t) * detail::kDecRows)),
       work_(new detail::Workspace()), gemm_work_(new detail::Workspace()),
       plan_(new detail::WorkList()),
-      inl_(new detail::InlineMeta()), rows_(new detail::DeviceRing()) {}
+      inl_(new detail::InlineMeta()) {}
 
 DecodeBatch::~DecodeBatch() = default;
 
@@ -500,7 +501,6 @@ Result<std::unique_ptr<DecodeBatch>> DecodeBatch::create(KVCacheManager &mgr, in
     const size_t n = static_cast<size_t>(max_seqs);
     const size_t words = 4 * n + 1 + 2 * (n + slots);
     batch->meta_->reserve(std::min<size_t>(words * 4, size_t(4) << 20));
-    batch->rows_->reserve(2 * sizeof(int32_t) * std::min<size_t>(n, detail::kDecRows));
     return R::ok(std::move(batch));
 }
 
@@ -755,7 +755,7 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
         rows.seq_row = d_rows_;
         rows.wpos = d_rows_ + n_;
     } else {
-        store = rows.store = rows_->next();
+        store = rows.store = meta_->next_tail();
     }
     detail::launch_w8a16(x, hidden, n_, hidden, group_size, segs, nseg, &rows, ws, stream, packed);
     if (store) {

@@ -91,26 +91,8 @@ bool stream_capturing(hipStream_t stream) {
     return true; // (the default stream beside a capture: the launch itself will report it)
 }
 
-// -------------------------------------------------------------- DeviceRing
-DeviceRing::~DeviceRing() {
-    if (base_) {
-        (void)hipDeviceSynchronize(); // kernels queued on callers' streams may still read it
-        (void)hipFree(base_);
-    }
-}
-
-void DeviceRing::reserve(size_t bytes) {
-    bytes_ = (bytes + 255) & ~size_t(255);
-    HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&base_), kSlots * bytes_));
-}
-
-int32_t *DeviceRing::next() {
-    cur_ = (cur_ + 1) % kSlots;
-    return reinterpret_cast<int32_t *>(base_ + static_cast<size_t>(cur_) * bytes_);
-}
-
 // ---------------------------------------------------------------- MetaRing
-MetaRing::MetaRing(int slots) : slots_(static_cast<size_t>(slots)) {}
+MetaRing::MetaRing(int slots, size_t tail) : slots_(static_cast<size_t>(slots)), tail_(tail) {}
 
 MetaRing::~MetaRing() {
     // kernels queued on callers' streams may still read the device slots
@@ -146,7 +128,7 @@ void MetaRing::grow(Slot &s, size_t bytes) {
     while (cap < bytes) cap <<= 1;
     void *host = nullptr, *dev = nullptr;
     HIP_CHECK(hipHostMalloc(&host, cap, hipHostMallocDefault));
-    HIP_CHECK(hipMalloc(&dev, cap));
+    HIP_CHECK(hipMalloc(&dev, cap + tail_));
     // The old host buffer is idle (its copy completed: begin() waited on the
     // slot's event); the old device buffer may still be read by queued kernels.
     if (s.host) retired_host_.push_back(s.host);
@@ -154,6 +136,12 @@ void MetaRing::grow(Slot &s, size_t bytes) {
     s.host = host;
     s.dev = dev;
     s.cap = cap;
+}
+
+int32_t *MetaRing::next_tail() {
+    tail_cur_ = (tail_cur_ + 1) % slots_.size();
+    const Slot &s = slots_[tail_cur_];
+    return reinterpret_cast<int32_t *>(static_cast<char *>(s.dev) + s.cap);
 }
 
 void MetaRing::reserve(size_t bytes) {

@@ -22,7 +22,8 @@ namespace detail {
 // memory next to the attention kernel and slowed it by more than it hid.)
 class MetaRing {
   public:
-    explicit MetaRing(int slots = 4);
+    // tail: bytes behind each slot's device buffer for kernels to fill (next_tail).
+    explicit MetaRing(int slots = 4, size_t tail = 0);
     ~MetaRing();
     MetaRing(const MetaRing &) = delete;
     MetaRing &operator=(const MetaRing &) = delete;
@@ -32,6 +33,10 @@ class MetaRing {
     // Sizes every slot for `bytes` now, so steps up to that size never
     // allocate.
     void reserve(size_t bytes);
+    // The tails in turn, after reserve(): what the first launch of a step brings
+    // in its arguments, kept for the step's further launches.  Ordered like the
+    // device buffers.
+    int32_t *next_tail();
 
   private:
     struct Slot {
@@ -49,26 +54,8 @@ class MetaRing {
     std::vector<void *> retired_dev_, retired_host_;
     int                 cur_ = -1;
     size_t              bytes_ = 0;
-};
-
-// Ring of equal device buffers that kernels fill: what the first launch of a
-// step brings in its arguments, kept for the step's further launches.  One
-// allocation, made by reserve(); a buffer is written again after three others,
-// in stream order behind the kernels that read it.
-class DeviceRing {
-  public:
-    DeviceRing() = default;
-    ~DeviceRing();
-    DeviceRing(const DeviceRing &) = delete;
-    DeviceRing &operator=(const DeviceRing &) = delete;
-    void     reserve(size_t bytes);
-    int32_t *next();
-
-  private:
-    static constexpr int kSlots = 4;
-    char  *base_ = nullptr;
-    size_t bytes_ = 0;
-    int    cur_ = 0;
+    const size_t        tail_;
+    size_t              tail_cur_ = 0;
 };
 
 // Whether work queued on the stream is being captured into a graph.

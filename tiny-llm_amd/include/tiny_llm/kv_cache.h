@@ -35,7 +35,6 @@ struct InlineMeta;
 struct PrefillEntry;
 struct PrefillInline;
 class MetaRing;
-class DeviceRing;
 class Workspace;
 } // namespace detail
 
@@ -216,9 +215,8 @@ class DecodeBatch {
     const int32_t  *d_part_base_ = nullptr, *d_work_ = nullptr;
     // Rows and positions that this prepare's first projection left in device
     // memory, on rows_stream_, for the next ones (null: none has yet).
-    std::unique_ptr<detail::DeviceRing> rows_;
-    const int32_t                      *d_rows_ = nullptr;
-    hipStream_t                         rows_stream_ = nullptr;
+    const int32_t  *d_rows_ = nullptr;
+    hipStream_t     rows_stream_ = nullptr;
 };
 
 // A prefill step over n sequences of one manager: sequence i brings

@@ -388,3 +388,90 @@ def test_prefill_plans_in_arguments_and_in_memory_agree(tl, paged):
         halves = 2 * (2 * n + 1) * 16 * H * D if paged else n * 2 * M * H * D
         pools.append(read_dev(g.pool(), halves))
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(pools[0], pools[1])
+
+
+def _steps(tl, L, H, Hq, D, n, paged, seed):
+    """A cache of n sequences with ragged prefixes, and per-step prompts."""
+    g = tl.KVCacheManager(L, H, D, 512, n, **(dict(block_tokens=16, num_blocks=32 * n) if paged else {}))
+    ids = [g.allocateSequence(512)[0] for _ in range(n)]
+    rng = np.random.default_rng(seed)
+    steps = []
+    for i in range(6):
+        order = rng.permutation(n)[:1 + 3 * i % n]
+        counts = [int(v) for v in rng.integers(1, 80, size=len(order))]
+        t = sum(counts)
+        steps.append((order, counts, to_dev(f16bits(rng, (t, Hq, D))), to_dev(f16bits(rng, (t, H * D))),
+                      to_dev(f16bits(rng, (t, H * D)))))
+    return g, ids, steps
+
+
+@pytest.mark.parametrize("paged,H,Hq,D", [(False, 2, 8, 64), (True, 2, 2, 128), (False, 1, 8, 256)])
+def test_prefill_every_layer_of_a_step(tl, paged, H, Hq, D):
+    """Layers after the first read the work that the first launch of the step
+    left on the device: outputs and cache are those of layers with a prepare of
+    their own, over steps of different order and size and on two streams."""
+    import torch
+    from devutil import read_dev
+    L, n = 4, 7
+    outs, pools = [], []
+    for own_prepare in (False, True):
+        g, ids, steps = _steps(tl, L, H, Hq, D, n, paged, 4)
+        pb = tl.PrefillBatch(g, n, Hq)
+        other = torch.cuda.Stream()
+        for i, (order, counts, q, k, v) in enumerate(steps):
+            seqs = [ids[j] for j in order]
+            for layer in range(L):
+                if layer == 0 or own_prepare:
+                    pb.prepare(seqs, counts, stream())
+                out = empty_dev(tuple(q.shape))
+                torch.cuda.synchronize()
+                st = other.cuda_stream if not own_prepare and i == 3 and layer in (1, 3) else stream()
+                if i == 4 and layer == 2:
+                    pb.append(layer, k.data_ptr(), v.data_ptr(), st)
+                    pb.attention(layer, q.data_ptr(), out.data_ptr(), D ** -0.5, st)
+                else:
+                    pb.run(layer, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), D ** -0.5, st)
+                outs.append(to_host(out))
+            pb.commit()
+        halves = 2 * (32 * n + 1) * 16 * H * D * L if paged else n * 2 * 512 * H * D * L
+        pools.append(read_dev(g.pool(), halves))
+    half = len(outs) // 2
+    for a, b in zip(outs[:half], outs[half:]):
+        assert np.array_equal(a, b)
+    assert np.array_equal(pools[0], pools[1])
+
+
+def test_prefill_replays_under_hip_graph_capture(tl):
+    """Layers of a step in a graph, with other steps between the replays: each
+    replay gives the outputs of the step it was captured from."""
+    import torch
+    L, H, Hq, D, n = 3, 2, 8, 64, 7
+    g, ids, steps = _steps(tl, L, H, Hq, D, n, False, 5)
+    pb = tl.PrefillBatch(g, n, Hq)
+    order, counts, q, k, v = steps[2]
+    outs = [empty_dev(tuple(q.shape)) for _ in range(L)]
+
+    def layers():
+        for layer in range(L):
+            pb.run(layer, q.data_ptr(), k.data_ptr(), v.data_ptr(), outs[layer].data_ptr(), D ** -0.5, stream())
+
+    pb.prepare([ids[j] for j in order], counts, stream())
+    layers()
+    want = [to_host(o) for o in outs]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layers()
+    torch.cuda.synchronize()
+    for rep in range(3):
+        for o, c, qq, kk, vv in steps[1:2] + steps[3:]:  # through every device buffer
+            pb.prepare([ids[j] for j in o], c, stream())
+            other = empty_dev(tuple(qq.shape))
+            for layer in range(L):
+                pb.run(layer, qq.data_ptr(), kk.data_ptr(), vv.data_ptr(), other.data_ptr(), D ** -0.5, stream())
+            torch.cuda.synchronize()
+        for o in outs:
+            o.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        assert all(np.array_equal(to_host(o), w) for o, w in zip(outs, want)), rep
+    del graph

@@ -106,3 +106,15 @@ def test_w8a16_dec_arguments(tmp_path):
     assert max(r["kernarg_segment_size"] for r in dec.values()) <= 384
     for name, r in rows.items():
         assert r["private_segment_fixed_size"] == 0 and r["vgpr_spill_count"] == 0, (name, r)
+
+
+def test_prefill_arguments(tmp_path):
+    """The work of a prefill step travels in the arguments of its first launch
+    only (3.6 KB, 0.4 us a launch); that form spills nothing either."""
+    ks = kernels("attention_prefill.o", tmp_path)
+    plain = {n: r for n, r in ks.items() if "attn_prefill_kernel" in n}
+    step = {n: r for n, r in ks.items() if "attn_prefill_step_kernel" in n}
+    assert len(plain) == len(step)
+    assert max(r["kernarg_segment_size"] for r in plain.values()) <= 256
+    bad = {n: r for n, r in step.items() if r["vgpr_spill_count"] or r["private_segment_fixed_size"]}
+    assert not bad, bad

@@ -48,6 +48,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <stdexcept>
+#include <type_traits>
 
 namespace tiny_llm {
 namespace detail {
@@ -111,7 +112,17 @@ struct PrefillArgs {
     const __half       *new_v;
     int                 Hkv;
     float               scale_log2;
-    PrefillInline       inl; // used when inl.n_entries > 0
+};
+
+// The first launch of a prepared step, its work in the arguments.  They cost a
+// launch 0.4 us, of which half is the second dependent load, so the kernel
+// leaves the records of `work` in device memory for the step's further layers;
+// these and the uniform launches keep the small arguments (a layer of one
+// prompt of 3 tokens 7.35 us with the work in every launch, 6.95 so; the legacy
+// entry point on 16 tokens 6.3 and 5.7).
+struct PrefillStepArgs : PrefillArgs {
+    PrefillInline inl;
+    int32_t      *store; // kPrefillItemWords words per item, or null
 };
 
 // Byte offsets of the token rows of one (cache row, kv head).
@@ -155,8 +166,10 @@ __device__ __forceinline__ uint4 ld16(const char *p) { return *reinterpret_cast<
 template <int D>
 constexpr int kQueryGroups = D <= 128 ? 2 : 1;
 
-template <int D, int G, bool PAGED, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void attn_prefill_kernel(PrefillArgs a) {
+// Args by value: through a reference they would be copied to scratch memory.
+template <int D, int G, bool PAGED, int NW, class Args>
+__device__ __forceinline__ void prefill_body(Args a) {
+    constexpr bool STEP = std::is_same_v<Args, PrefillStepArgs>;
     static_assert(D == 32 || D == 64 || D == 128 || D == 256, "head_dim");
     static_assert(G == 1 || G == 2 || G == 4 || G == 8, "group size");
     static_assert(NW == 4 || (NW == 8 && D <= 128), "waves");
@@ -196,7 +209,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 12
     const int g = blockIdx.x - item * a.Hkv;
     int64_t   q_off;
     int       p0, n, row, qt, tok0 = 0;
-    if (a.inl.n_entries) {
+    if constexpr (STEP) {
         const uint32_t it = (uint32_t)a.inl.w[4 * a.inl.n_entries + item];
         const int      e = 4 * (int)(it >> 16);
         p0 = a.inl.w[e];
@@ -521,18 +534,45 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 12
             *reinterpret_cast<uint4 *>(a.out + o) = *reinterpret_cast<const uint4 *>(&stg[rr * OP + 8 * pc]);
         }
     }
+    if constexpr (STEP) { // (at the end: nothing waits for these)
+        if (a.store && g == 0 && tid == 0) {
+            const uint64_t qo = (uint64_t)q_off;
+            int4          *w = reinterpret_cast<int4 *>(a.store + (int64_t)kPrefillItemWords * item);
+            w[0] = make_int4((int)(uint32_t)qo, (int)(qo >> 32), p0, n);
+            w[1] = make_int4(row, qt, tok0, 0);
+        }
+    }
+}
+
+#define TL_PREFILL_BOUNDS(D, NW) __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1)))
+
+template <int D, int G, bool PAGED, int NW>
+__global__ TL_PREFILL_BOUNDS(D, NW) void attn_prefill_kernel(PrefillArgs a) {
+    prefill_body<D, G, PAGED, NW>(a);
+}
+
+template <int D, int G, bool PAGED, int NW>
+__global__ TL_PREFILL_BOUNDS(D, NW) void attn_prefill_step_kernel(PrefillStepArgs a) {
+    prefill_body<D, G, PAGED, NW>(a);
 }
 
 template <int D, int G, int NW>
-void launch_dgw(const PrefillArgs &a, int grid, bool paged, hipStream_t stream) {
-    if (paged)
-        hipLaunchKernelGGL((attn_prefill_kernel<D, G, true, NW>), dim3(grid), dim3(NW * 64), 0, stream, a);
-    else
-        hipLaunchKernelGGL((attn_prefill_kernel<D, G, false, NW>), dim3(grid), dim3(NW * 64), 0, stream, a);
+void launch_dgw(const PrefillStepArgs &a, int grid, bool paged, hipStream_t stream) {
+    const PrefillArgs &small = a;
+#define TL_PREFILL_LAUNCH(P)                                                                                          \
+    do {                                                                                                              \
+        if (a.inl.n_entries)                                                                                          \
+            hipLaunchKernelGGL((attn_prefill_step_kernel<D, G, P, NW>), dim3(grid), dim3(NW * 64), 0, stream, a);     \
+        else                                                                                                          \
+            hipLaunchKernelGGL((attn_prefill_kernel<D, G, P, NW>), dim3(grid), dim3(NW * 64), 0, stream, small);      \
+    } while (0)
+    if (paged) TL_PREFILL_LAUNCH(true);
+    else TL_PREFILL_LAUNCH(false);
+#undef TL_PREFILL_LAUNCH
 }
 
 template <int D, int G>
-void launch_dg(const PrefillArgs &a, int grid, int waves, bool paged, hipStream_t stream) {
+void launch_dg(const PrefillStepArgs &a, int grid, int waves, bool paged, hipStream_t stream) {
     if constexpr (D <= 128) {
         if (waves == 8) {
             launch_dgw<D, G, 8>(a, grid, paged, stream);
@@ -543,7 +583,7 @@ void launch_dg(const PrefillArgs &a, int grid, int waves, bool paged, hipStream_
 }
 
 template <int D>
-void launch_d(const PrefillArgs &a, int grid, int G, int waves, bool paged, hipStream_t stream) {
+void launch_d(const PrefillStepArgs &a, int grid, int G, int waves, bool paged, hipStream_t stream) {
     switch (G) {
     case 1: launch_dg<D, 1>(a, grid, waves, paged, stream); break;
     case 2: launch_dg<D, 2>(a, grid, waves, paged, stream); break;
@@ -680,7 +720,7 @@ void launch_attn_prefill(const PrefillLaunch &p, const KvView &kv, int Hq, int H
         items = p.uniform_b * ((p.uniform_n + BQ - 1) / BQ);
     }
     if (items <= 0) return;
-    PrefillArgs a;
+    PrefillStepArgs a;
     a.q = p.q;
     a.out = p.out;
     a.kv = kv;
@@ -690,6 +730,7 @@ void launch_attn_prefill(const PrefillLaunch &p, const KvView &kv, int Hq, int H
     a.q_entry = p.q_entry_stride;
     a.uniform_b = p.uniform_b;
     a.uniform_n = p.uniform_n;
+    a.store = p.store;
     if (p.inl) a.inl = *p.inl;
     else a.inl.n_entries = 0;
     if ((p.new_k != nullptr) != (p.new_v != nullptr) || (p.new_k && !p.work && !p.inl))

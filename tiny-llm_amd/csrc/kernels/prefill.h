@@ -101,8 +101,10 @@ struct PrefillLaunch {
     const int32_t      *work = nullptr;
     int                 n_items = 0;
     int                 waves = 0;
-    // ... or the same in the kernel arguments (with `waves`) ...
+    // ... or the same in the kernel arguments (with `waves`), left in `store`
+    // (device memory, may be null) as the items of `work` ...
     const PrefillInline *inl = nullptr;
+    int32_t             *store = nullptr;
     // ... or, with neither, `uniform_b` entries b with p0 = 0,
     // n = uniform_n, row = b and q_off = b * q_entry_stride (waves by
     // prefill_waves_uniform).

@@ -771,7 +771,8 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
 
 PrefillBatch::PrefillBatch(KVCacheManager &mgr, int max_seqs, int num_q_heads)
     : mgr_(mgr), max_seqs_(max_seqs), num_q_heads_(num_q_heads), meta_(new detail::MetaRing(4)),
-      inl_(new detail::PrefillInline) {}
+      inl_(new detail::PrefillInline),
+      records_(new detail::DeviceRing(sizeof(int32_t) * detail::kPrefillItemWords * detail::kPrefillInlineWords)) {}
 
 PrefillBatch::~PrefillBatch() = default;
 
@@ -801,6 +802,7 @@ Result<void> PrefillBatch::prepare(const int *seq_ids, const int *num_tokens, in
     d_work_ = nullptr;
     uploaded_ = false;
     inline_ok_ = false;
+    launched_ = false;
     ids_.clear();
     counts_.clear();
     slots_.clear();
@@ -913,21 +915,33 @@ Result<void> PrefillBatch::launch(int layer_idx, const half *q, const half *new_
          reinterpret_cast<uintptr_t>(new_k) | reinterpret_cast<uintptr_t>(new_v)) & 15u)
         return Result<void>::err("PrefillBatch: q, out, new_k and new_v must be 16-byte aligned");
     if (n_items_ == 0) return Result<void>::ok();
-    if (!inline_ok_) upload_device(stream);
     detail::PrefillLaunch p;
+    if (!inline_ok_) {
+        upload_device(stream);
+    } else {
+        // A captured launch carries its work: replays then depend on nothing
+        // that later steps rewrite.
+        const bool captured = detail::stream_capturing(stream);
+        if (captured || !d_work_ || work_stream_ != stream) p.inl = inl_.get();
+        if (!captured && p.inl && (launched_ || records_->allocated())) p.store = records_->next();
+        launched_ = true;
+    }
     p.q = q;
     p.out = out;
     p.q_tok_stride = static_cast<int64_t>(num_q_heads_) * cfg.head_dim;
     p.q_head_stride = cfg.head_dim;
-    p.work = d_work_;
+    p.work = p.inl ? nullptr : d_work_;
     p.n_items = n_items_;
-    p.inl = inline_ok_ ? inl_.get() : nullptr;
     p.waves = waves_;
     p.max_keys = max_keys_;
     p.new_k = new_k;
     p.new_v = new_v;
     detail::launch_attn_prefill(p, mgr_.layerView(layer_idx, nullptr), num_q_heads_, cfg.num_heads,
                                 cfg.head_dim, scale, stream);
+    if (p.store) {
+        d_work_ = p.store;
+        work_stream_ = stream;
+    }
     return Result<void>::ok();
 }
 

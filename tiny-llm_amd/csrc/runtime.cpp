@@ -91,6 +91,20 @@ bool stream_capturing(hipStream_t stream) {
     return true; // (the default stream beside a capture: the launch itself will report it)
 }
 
+// -------------------------------------------------------------- DeviceRing
+DeviceRing::~DeviceRing() {
+    if (base_) {
+        (void)hipDeviceSynchronize(); // kernels queued on callers' streams may still read it
+        (void)hipFree(base_);
+    }
+}
+
+int32_t *DeviceRing::next() {
+    if (!base_) HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&base_), kSlots * bytes_));
+    cur_ = (cur_ + 1) % kSlots;
+    return reinterpret_cast<int32_t *>(base_ + static_cast<size_t>(cur_) * bytes_);
+}
+
 // ---------------------------------------------------------------- MetaRing
 MetaRing::MetaRing(int slots, size_t tail) : slots_(static_cast<size_t>(slots)), tail_(tail) {}
 

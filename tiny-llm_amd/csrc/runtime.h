@@ -58,6 +58,26 @@ class MetaRing {
     size_t              tail_cur_ = 0;
 };
 
+// Ring of four equal device buffers that kernels fill: what the first launch
+// of a step brings in its arguments, kept for the step's further launches.  One
+// allocation, at the first next(); a buffer is written again after three others,
+// in stream order behind the kernels that read it.
+class DeviceRing {
+  public:
+    explicit DeviceRing(size_t bytes) : bytes_((bytes + 255) & ~size_t(255)) {}
+    ~DeviceRing();
+    DeviceRing(const DeviceRing &) = delete;
+    DeviceRing &operator=(const DeviceRing &) = delete;
+    bool     allocated() const { return base_ != nullptr; }
+    int32_t *next();
+
+  private:
+    static constexpr int kSlots = 4;
+    char        *base_ = nullptr;
+    const size_t bytes_;
+    int          cur_ = 0;
+};
+
 // Whether work queued on the stream is being captured into a graph.
 bool stream_capturing(hipStream_t stream);
 

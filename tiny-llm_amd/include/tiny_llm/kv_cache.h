@@ -35,6 +35,7 @@ struct InlineMeta;
 struct PrefillEntry;
 struct PrefillInline;
 class MetaRing;
+class DeviceRing;
 class Workspace;
 } // namespace detail
 
@@ -276,9 +277,14 @@ class PrefillBatch {
     std::unique_ptr<detail::MetaRing> meta_;
     const int32_t       *d_work_ = nullptr;
     // The work in the kernel arguments where it fits (then work_ is empty and
-    // nothing is uploaded).
+    // nothing is uploaded): the first launch of a prepared step leaves it in
+    // device memory (d_work_), for the next ones on the same stream.  (Until a
+    // step has a second layer there is no such memory.)
     std::unique_ptr<detail::PrefillInline> inl_;
     bool                                   inline_ok_ = false;
+    std::unique_ptr<detail::DeviceRing>    records_;
+    hipStream_t                            work_stream_ = nullptr;
+    bool                                   launched_ = false;
 };
 
 } // namespace tiny_llm

@@ -347,6 +347,13 @@ int tl_w8a16_pack(const int8_t *weight, int K, int N, int8_t *packed, void *stre
  * allows), 1 = always the reference-order kernel.  No reference counterpart
  * (test knob). */
 int tl_w8a16_set_path(int path);
+/* The kernel that an M x N x K product with 16-byte aligned operands runs with
+ * path 0 on num_cus CUs (0: the current device's): 0 = reference order, 1 =
+ * decode sizes, 2 = split-K, 3 = tiles of tile_rows x tile_cols outputs (0 x 0 for
+ * the others; the tile may depend on `packed`, the kernel does not).  No
+ * reference counterpart. */
+int tl_w8a16_plan(int M, int N, int K, int group_size, int packed, int num_cus, int *kernel,
+                  int *tile_rows, int *tile_cols);
 
 /* Score (q.K^T) path of the decode attention kernels, process-wide:
  * 0 = VALU v_dot2 over the loaded K rows, 1 = MFMA v_mfma_f32_16x16x32_f16

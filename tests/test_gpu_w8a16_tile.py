@@ -48,6 +48,41 @@ def test_w8a16_tile_edges(tl, orc, M, N, K, gs):
     assert np.array_equal(np.where(got == 0x8000, 0, got), got_p)
 
 
+# Every tile of the kernel in both layouts, at the edges of its rows, columns, K
+# chunks, K halves and scale groups: (M, N, K, group size), the tile with
+# row-major weights and with packed ones.
+TILE_SHAPES = [
+    ((641, 9232, 32, 64), (128, 256), (128, 256)),     # one row over; one k step: no chunk at all
+    ((257, 16400, 64, 64), (128, 256), (64, 128)),     # one chunk: the second K half is empty; several rounds
+    ((2048, 4096, 96, 256), (128, 256), (128, 256)),   # full tiles, an unpaired last step, a group longer than K
+    ((641, 9232, 160, 128), (128, 256), (128, 256)),   # a partial last group
+    ((2047, 4080, 1056, 128), (128, 256), (128, 256)), # rows and columns short of the last tile, groups over chunks
+    ((585, 8208, 160, 128), (128, 192), (128, 192)),
+    ((65, 24592, 96, 128), (128, 128), (128, 128)),    # 63 rows of padding
+    ((129, 16400, 288, 64), (64, 256), (64, 256)),     # K % 64 == 32 inside a group
+    ((65, 16400, 2080, 512), (64, 192), (64, 192)),    # a group over the boundary of the K halves
+    ((65, 12304, 1056, 512), (64, 128), (64, 128)),
+    ((9250, 1008, 192, 256), (128, 192), (64, 128)),   # more row tiles than a panel
+    ((200, 16400, 1056, 32), (128, 192), (128, 192)),  # two groups per chunk, from here
+    ((65, 24592, 1120, 32), (128, 128), (128, 128)),
+    ((129, 16400, 1056, 32), (64, 256), (64, 256)),
+    ((65, 18608, 1056, 32), (64, 192), (64, 192)),
+    ((129, 9232, 1056, 32), (64, 128), (64, 128)),
+]
+
+
+@pytest.mark.parametrize("shape,tile,tile_packed", TILE_SHAPES)
+def test_w8a16_every_tile(tl, orc, shape, tile, tile_packed):
+    M, N, K, gs = shape
+    assert tl.w8a16_plan(*shape) == ("tile", *tile) and tl.w8a16_plan(*shape, packed=True) == ("tile", *tile_packed)
+    rng = np.random.default_rng(M + 3 * N + 7 * K + gs)
+    x, w, s = operands(orc, rng, M, N, K, gs)
+    ref = product(x, w, s, K, gs)
+    got, got_p = both(tl, to_dev(x), w, to_dev(s), M, N, K, gs)
+    assert rows_close(got, ref) <= TOL
+    assert np.array_equal(np.where(got == 0x8000, 0, got), got_p)
+
+
 def test_w8a16_tile_scales(tl, orc):
     """Zero scales (whole columns, first, middle and last groups), negative and
     subnormal ones, and scales far apart."""
@@ -120,10 +155,36 @@ def test_w8a16_tile_unaligned_output(tl, orc):
     assert np.array_equal(got[1:-1], to_host(out).reshape(-1)) and got[0] == got[-1] == 0x3555
 
 
+def test_w8a16_tile_element_stores(tl, orc):
+    """As above where the tile kernel writes the outputs."""
+    M, N, K, gs = 585, 8208, 160, 128
+    assert tl.w8a16_plan(M, N, K, gs)[0] == "tile"
+    rng = np.random.default_rng(14)
+    x, w, s = operands(orc, rng, M, N, K, gs)
+    dx, dw, ds = to_dev(x), to_dev_raw(w), to_dev(s)
+    out, off = empty_dev((M, N)), to_dev(np.full(M * N + 2, 0x3555, np.uint16))
+    tl.w8a16_matmul(dx.data_ptr(), dw.data_ptr(), ds.data_ptr(), out.data_ptr(), M, N, K, gs, stream())
+    tl.w8a16_matmul(dx.data_ptr(), dw.data_ptr(), ds.data_ptr(), off.data_ptr() + 2, M, N, K, gs, stream())
+    got = to_host(off)
+    assert np.array_equal(got[1:-1], to_host(out).reshape(-1)) and got[0] == got[-1] == 0x3555
+
+
+@pytest.mark.parametrize("paged,B,Hkv,kernels", [
+    (False, 650, 16, ("tile", "split-k")),  # q, and k and v
+    (True, 650, 16, ("tile", "split-k")),
+    (False, 1200, 32, ("tile", "tile")),
+    (True, 1200, 32, ("tile", "tile")),
+])
+def test_project_tiles_equal_products(tl, orc, paged, B, Hkv, kernels):
+    """The projections whose q part, or all parts, run in the tile kernel."""
+    assert tuple(tl.w8a16_plan(B, n * 128, 320, 64)[0] for n in (4 * Hkv, Hkv)) == kernels
+    test_project_large_batch_equals_products(tl, orc, paged, B, Hkv, 128)
+
+
 @pytest.mark.parametrize("paged,B,Hkv,D", [
     (False, 130, 2, 64),    # all columns to the split-K kernel
-    (True, 650, 8, 128),    # q to the tile kernel, k and v to the split-K one
-    (False, 1200, 8, 256),  # all to the tile kernel
+    (True, 650, 8, 128),    # as the first, with more columns
+    (False, 1200, 8, 256),  # q to the tile kernel, k and v to the split-K one
     (True, 1200, 8, 256),
 ])
 def test_project_large_batch_equals_products(tl, orc, paged, B, Hkv, D):

@@ -4,6 +4,7 @@
 
 #include "kernels/kv_kernels.h"
 #include "kernels/prefill.h"
+#include "kernels/w8a16.h"
 #include "runtime.h"
 #include "tiny_llm/kernels/attention.h"
 #include "tiny_llm/kv_cache.h"
@@ -389,6 +390,21 @@ int tl_w8a16_set_path(int path) {
     tiny_llm::detail::w8a16_force_generic(path);
     g_last_error.clear();
     return TL_OK;
+}
+
+int tl_w8a16_plan(int M, int N, int K, int group_size, int packed, int num_cus, int *kernel,
+                  int *tile_rows, int *tile_cols) {
+    namespace d = tiny_llm::detail;
+    if (!kernel || !tile_rows || !tile_cols) return fail(TL_ERR_INVALID, "tl_w8a16_plan: null result");
+    if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || num_cus < 0)
+        return fail(TL_ERR_INVALID, "tl_w8a16_plan: sizes must be positive");
+    return guarded([&] {
+        const d::W8A16Plan p = d::w8a16_plan(M, N, K, group_size, packed != 0, num_cus > 0 ? num_cus : d::device_cus());
+        *kernel = static_cast<int>(p.kernel);
+        *tile_rows = p.rows;
+        *tile_cols = p.cols;
+        return TL_OK;
+    });
 }
 
 void tl_attention_decode(const void *q, const void *k, const void *v, void *out, float scale,

@@ -62,6 +62,15 @@ bool w8a16_mfma_ok(int K, int gs, const W8A16Seg *segs, int nseg);
 // for the segments that w8a16_tile_kernel does not take.
 size_t w8a16_workspace_floats(int M, int K, int gs, const W8A16Seg *segs, int nseg);
 
+// The kernel that a product of one matrix with aligned operands runs on `cus` CUs,
+// and the tile of the tile kernel.
+enum class W8A16Kernel { Generic, Dec, SplitK, Tile };
+struct W8A16Plan {
+    W8A16Kernel kernel = W8A16Kernel::Generic;
+    int         rows = 0, cols = 0;
+};
+W8A16Plan w8a16_plan(int M, int N, int K, int gs, bool packed, int cus);
+
 // True when launch_w8a16 will run w8a16_dec_kernel for these operands.
 bool w8a16_takes_dec(const __half *x, int64_t ldx, int M, int K, int gs, const W8A16Seg *segs, int nseg, bool packed);
 

@@ -51,6 +51,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <stdexcept>
 #include <string>
@@ -1516,40 +1517,30 @@ DecPlan dec_plan(int M, int gs, const W8A16Seg *segs, int nseg) {
 } // namespace
 
 namespace {
-// A segment of n columns goes to w8a16_tile_kernel by its own size, never by
-// what shares the call, so that the fused projection's bytes equal the separate
-// products'.  Its smallest tiles still walk K in steps of about 0.6 us, two
-// K halves at a time (27 us for K = 4096, however few the tiles), so it takes
-// the outputs that keep the split-K kernel busy longer than that.  Row-major /
-// packed us, split-K -> tile, K = 4096: 512 x 4096 32.2 / 32.0 -> 33.2 / 28.5
-// and 1536 x 1024 30.9 / 31.1 -> 32.3 / 27.6 (both left alone), 300 x 8192
-// 47.7 / 47.2 -> 45.2 / 37.2, 8192 x 256 45.1 / 47.3 -> 33.1 / 28.9; K = 14336:
-// 600 x 4096 138.6 / 127.1 -> 138.8 / 110.5.  Up to 256 rows the split-K kernel
-// also writes and sums partials when K is 2048 or more: 128 x 11008 40.2 / 39.3
-// -> 32.5 / 27.3, 256 x 8192 54.1 / 53.8 -> 32.9 / 28.8 (but K = 512, 192 x
-// 11008: 10.6 / 11.5 -> 12.1 / 11.2).  Between 256 and 640 rows and up to 8192
-// columns, where the matrix may be the q part of a decode batch's projection
-// whose k and v parts stay with the split-K kernel, it has to win more than the
-// second launch costs (packed, prepare + project: 350 x (8192 + 2 x 1024) 102 ->
-// 112 us, 580 x (4096 + 2 x 1024) 61 -> 73, both left alone; 600 x (8192 + 2 x
-// 1024) 167 -> 150).
-bool tile_ok(int M, int n, int K) {
-    const int64_t outputs = (int64_t)M * n;
-    if (M <= 64) return false;
-    if (M <= 256 && K >= 2048) return outputs >= 5LL << 18;
-    return outputs >= (M > 256 && M <= 640 && n <= 8192 ? 17LL << 18 : 9LL << 18);
+// Plan of w8a16_tile_kernel: the tile shape whose rounds of one workgroup per CU
+// take least, by the measured time of a round (the larger tile on a tie).  The
+// shape may differ between the layouts: it does not touch the results.
+struct TilePlan {
+    int   rb = 8, cb = 4, rtiles = 0, ctiles = 0;
+    float us = 0.0f;
+};
+
+// `rounds` rounds of RB x CB tiles: (K + 850) times the ns below, the 850 for the
+// launch, the first loads, the exchange of the K halves and the output.  Measured
+// at six K from 512 to 14336 and one to four rounds, within 6%; K = 4096, groups of
+// 128: 64 x 128 / 192 / 256 tiles 34 / 47 / 58 us row-major and 28 / 38 / 46
+// packed, 128 x 128 / 192 / 256 48 / 64 / 77 and 43 / 56 / 70.  Two packed 64 x 128
+// workgroups fit a CU, so that their further rounds add 20 us, not 28.  Groups of
+// 32 rescale twice a chunk and take a third more.
+float tile_us(int rb, int cb, int64_t rounds, int K, int gs, bool packed) {
+    static constexpr float kNs[2][2][3] = {{{6.9f, 9.4f, 11.8f}, {9.8f, 12.9f, 15.6f}},
+                                           {{5.7f, 7.7f, 9.4f}, {8.6f, 11.3f, 14.2f}}};
+    const float r = packed && rb == 4 && cb == 2 ? 0.3f + 0.7f * (float)rounds : (float)rounds;
+    return r * kNs[packed][rb / 4 - 1][cb - 2] * 1e-3f * (float)(K + 850) * (gs == 32 ? 1.3f : 1.0f);
 }
 
-// Plan of w8a16_tile_kernel: the tile shape with the least padded work in the
-// longest CU's share, (rounds of one workgroup per CU) x RB x CB, the larger
-// tile on a tie (its x and weight traffic per product is the lowest).
-struct TilePlan {
-    int rb = 8, cb = 4, rtiles = 0, ctiles = 0;
-};
-TilePlan tile_plan(int M, int gs, const W8A16Seg *segs, int nseg) {
-    TilePlan  best;
-    int64_t   cost = INT64_MAX;
-    const int cus = std::max(1, device_cus());
+TilePlan tile_plan(int M, int K, int gs, const W8A16Seg *segs, int nseg, bool packed, int cus) {
+    TilePlan best;
     for (int rb = 8; rb >= 4; rb -= 4)
         for (int cb = 4; cb >= 2; --cb) {
             if (gs == 32 && rb == 8 && cb == 4) continue; // two scales per chunk do not fit its registers
@@ -1558,13 +1549,40 @@ TilePlan tile_plan(int M, int gs, const W8A16Seg *segs, int nseg) {
             p.cb = cb;
             p.rtiles = (M + 16 * rb - 1) / (16 * rb);
             for (int i = 0; i < nseg; ++i) p.ctiles += (segs[i].n + 64 * cb - 1) / (64 * cb);
-            const int64_t rounds = ((int64_t)p.rtiles * p.ctiles + cus - 1) / cus;
-            if (rounds * rb * cb < cost) {
-                cost = rounds * rb * cb;
-                best = p;
-            }
+            p.us = tile_us(rb, cb, ((int64_t)p.rtiles * p.ctiles + cus - 1) / cus, K, gs, packed);
+            if (!best.rtiles || p.us < best.us) best = p;
         }
     return best;
+}
+
+// A segment goes to w8a16_tile_kernel by its own size, never by what shares the
+// call or by the weight layout, so that the fused projection's bytes equal the
+// separate products' and both layouts give the same bits: by the times of packed
+// weights, where the two kernels are nearest.  The split-K kernel takes 2.2 us + K *
+// 2.65 ns for each 64 x 64 tile that a CU gets, whole tiles, and up to 256 rows,
+// where K is split and partials are written and summed, 2.5 us + K * 4.7 ns per
+// tile and CU (groups below 128, with their second accumulator, 10 and 25%
+// more).  The margin is for row-major weights, which lose more with a short K, and
+// with groups of 32 up to 256 rows.
+//
+// Measured on 2900 products (K 512 .. 14336, 80 .. 4096 rows, both layouts) and 378
+// projections of 65 .. 2048 entries, against the split-K kernel alone.  A bound
+// on the outputs (9 * 2^18) and a tile plan by its padded work, which these
+// replace, made 146 products slower, by up to 40% (1152 x 8192 x 512 row-major 33
+// -> 46 us), and 34 projections, whose k and v parts stay with the split-K kernel in
+// a second launch, by up to 38% (1152 x (2048 + 2 x 256) x 2048 row-major 31 -> 43).
+// These make no product slower, and 9 projections, by up to 15% (1152 x
+// (4096 + 2 x 512) x 2048 row-major 50 -> 57; the q part alone 48 -> 37): a rule that
+// spares those too leaves 13% of the products at up to twice their time.
+bool tile_ok(int M, int K, int gs, const W8A16Seg &seg, int cus) {
+    if (M <= kDecRows) return false;
+    const float tiles = (float)((M + kBM - 1) / kBM) * (float)((seg.n + kBN - 1) / kBN) / (float)cus;
+    const bool  split = M <= 256 && K >= 1024;
+    const float sk = split ? (tiles + 0.2f) * (2.5f + 4.7e-3f * (float)K) * (gs < 128 ? 1.25f : 1.0f)
+                           : std::ceil(tiles) * (2.2f + 2.65e-3f * (float)K) * (gs < 128 ? 1.1f : 1.0f);
+    const float bar = sk / (K < 1024 || (split && gs == 32) ? 1.2f : 1.08f);
+    if (tile_us(4, 2, 1, K, gs, true) > bar) return false; // (the least there is: no plan for small products)
+    return tile_plan(M, K, gs, &seg, 1, true, cus).us <= bar;
 }
 
 void launch_tile(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
@@ -1572,7 +1590,7 @@ void launch_tile(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
     std::memset(&a, 0, sizeof(a));
     a.g = g;
     a.log2_spg = __builtin_ctz((unsigned)(gs / 32));
-    const TilePlan p = tile_plan(g.M, gs, g.seg, g.nseg);
+    const TilePlan p = tile_plan(g.M, g.K, gs, g.seg, g.nseg, packed, std::max(1, device_cus()));
     a.rtiles = p.rtiles;
     a.ctiles = p.ctiles;
     a.panel = p.rtiles <= 6 ? p.rtiles : 4;
@@ -1614,10 +1632,29 @@ void launch_tile(const GemmArgs &g, int gs, hipStream_t stream, bool packed) {
 }
 } // namespace
 
+W8A16Plan w8a16_plan(int M, int N, int K, int gs, bool packed, int cus) {
+    W8A16Seg seg;
+    seg.n = N;
+    W8A16Plan out;
+    if (!w8a16_mfma_ok(K, gs, &seg, 1)) return out;
+    if (dec_ok(M, K, &seg, 1)) {
+        out.kernel = W8A16Kernel::Dec;
+    } else if (tile_ok(M, K, gs, seg, cus)) {
+        const TilePlan t = tile_plan(M, K, gs, &seg, 1, packed, cus);
+        out.kernel = W8A16Kernel::Tile;
+        out.rows = 16 * t.rb;
+        out.cols = 64 * t.cb;
+    } else {
+        out.kernel = W8A16Kernel::SplitK;
+    }
+    return out;
+}
+
 size_t w8a16_workspace_floats(int M, int K, int gs, const W8A16Seg *segs, int nseg) {
     if (!w8a16_mfma_ok(K, gs, segs, nseg) || dec_ok(M, K, segs, nseg)) return 0;
-    int ntot = 0;
-    for (int i = 0; i < nseg; ++i) ntot += tile_ok(M, segs[i].n, K) ? 0 : segs[i].n;
+    const int cus = std::max(1, device_cus());
+    int       ntot = 0;
+    for (int i = 0; i < nseg; ++i) ntot += tile_ok(M, K, gs, segs[i], cus) ? 0 : segs[i].n;
     const int splits = split_plan(M, K, nullptr);
     return splits > 1 ? (size_t)splits * M * ntot : 0;
 }
@@ -1750,8 +1787,9 @@ void launch_w8a16(const __half *x, int64_t ldx, int M, int K, int gs, const W8A1
     GemmArgs big = a;
     big.nseg = a.nseg = 0;
     tiles = 0;
+    const int cus = std::max(1, device_cus());
     for (int i = 0; i < nseg; ++i) {
-        GemmArgs &to = tile_ok(M, segs[i].n, K) ? big : a;
+        GemmArgs &to = tile_ok(M, K, gs, segs[i], cus) ? big : a;
         to.seg[to.nseg] = segs[i];
         to.col0[to.nseg + 1] = to.col0[to.nseg] + segs[i].n;
         ++to.nseg;

@@ -140,6 +140,7 @@ def _declare(L: C.CDLL) -> None:
         "tl_w8a16_matmul": (i, [vp, vp, vp, vp, i, i, i, i, vp]),
         "tl_w8a16_matmul_residual": (i, [vp, vp, vp, vp, i, i, i, i, i, vp]),
         "tl_w8a16_set_path": (i, [i]),
+        "tl_w8a16_plan": (i, [i, i, i, i, i, i, ip, ip, ip]),
         "tl_attn_decode_gqa": (i, [vp, C.POINTER(KVView), vp, i, i, i, i, f, vp, vp]),
         "tl_attn_decode_gqa_noalloc": (i, [vp, C.POINTER(KVView), vp, i, i, i, i, f, vp, vp]),
         "tl_attn_noalloc_scratch_bytes": (sz, []),
@@ -630,3 +631,15 @@ def w8a16_pack(weight, K, N, packed, stream=0):
 def w8a16_set_path(path: int):
     """0 = MFMA where the shape allows, 1 = always the reference-order kernel."""
     _check(load().tl_w8a16_set_path(path))
+
+
+_W8A16_KERNELS = ("reference", "decode", "split-k", "tile")
+
+
+def w8a16_plan(M, N, K, group_size, packed=False, num_cus=0):
+    """(kernel, tile rows, tile columns) of a product with aligned operands;
+    num_cus 0 = the current device's.  Kernels: "reference", "decode", "split-k"
+    and "tile"; the tile is (0, 0) for the others."""
+    k, r, c = C.c_int(0), C.c_int(0), C.c_int(0)
+    _check(load().tl_w8a16_plan(M, N, K, group_size, int(packed), num_cus, C.byref(k), C.byref(r), C.byref(c)))
+    return _W8A16_KERNELS[k.value], r.value, c.value

@@ -7,7 +7,7 @@ release / re-allocate (stale bytes included) and paged block maps."""
 import numpy as np
 import pytest
 
-from devutil import read_dev, stream, to_dev, to_host
+from devutil import empty_dev, read_dev, stream, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -286,3 +286,63 @@ def test_gather_metadata_forms(tl, n, paged, which):
             m = min(lens[i], s_max)
             rows = src[at[i]:at[i] + m].reshape(m, H, D).transpose(1, 0, 2)
             assert np.array_equal(got[b, :, :m], rows) and not got[b, :, m:].any()
+
+
+@pytest.mark.parametrize("paged", [False, True])
+def test_gather_every_layer_of_a_step(tl, paged):
+    """Layers after the first read the lengths and rows that the step's first
+    gather left on the device: over steps of different order and size, on two
+    streams, beside projections' rows, and in a graph that is replayed after
+    further steps."""
+    import torch
+    L, H, D, M, n = 3, 2, 32, 48, 70
+    rng = np.random.default_rng(21)
+    g = tl.KVCacheManager(L, H, D, M, n, **(dict(block_tokens=16, num_blocks=3 * n) if paged else {}))
+    lens = [int(v) for v in rng.integers(1, M, size=n)]
+    at = np.concatenate([[0], np.cumsum(lens)])
+    kv = [[rng.standard_normal((at[-1], H * D)).astype(np.float16).view(np.uint16) for _ in range(2)] for _ in range(L)]
+    ids = [g.allocateSequence(M)[0] for _ in range(n)]
+    pb = tl.PrefillBatch(g, n, H)
+    pb.prepare(ids, lens, stream())
+    keep = [[to_dev(t) for t in layer] for layer in kv]
+    for layer, (k, v) in enumerate(keep):
+        pb.append(layer, k.data_ptr(), v.data_ptr(), stream())
+    pb.commit()
+    batch = tl.DecodeBatch(g, n, H)
+    outs = [[empty_dev((n, H, M, D)) for _ in range(2)] for _ in range(L)]
+
+    def gather(layer, st, both=True):
+        batch.gather(layer, outs[layer][0].data_ptr(), outs[layer][1].data_ptr() if both else 0, M, st)
+
+    def check(layer, order, cut, both=True):
+        for w in range(1 + both):
+            got = to_host(outs[layer][w])
+            for b, i in enumerate(order):
+                m = min(lens[i], cut)
+                rows = kv[layer][w][at[i]:at[i] + m].reshape(m, H, D).transpose(1, 0, 2)
+                assert np.array_equal(got[b, :, :m], rows) and not got[b, :, m:].any()
+
+    def prepare(step):
+        order, cut = rng.permutation(n)[:1 + 23 * step % n], int(rng.integers(1, M))
+        batch.prepare_lengths([ids[i] for i in order], [min(lens[i], cut) for i in order], stream())
+        return order, cut
+
+    other, graph, captured = torch.cuda.Stream(), torch.cuda.CUDAGraph(), None
+    for step in range(9):  # more steps than device buffers
+        order, cut = prepare(step)
+        torch.cuda.synchronize()
+        for layer in range(L):
+            both = step != 2
+            gather(layer, other.cuda_stream if step == 4 and layer == 1 else stream(), both)
+            torch.cuda.synchronize()
+            check(layer, order, cut, both)
+        if step == 3:
+            with torch.cuda.graph(graph):
+                for layer in range(L):
+                    gather(layer, stream())
+            captured = order, cut
+        if captured and step > 5:
+            graph.replay()
+            for layer in range(L):
+                check(layer, *captured)
+    del graph

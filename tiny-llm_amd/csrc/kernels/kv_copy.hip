@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 namespace tiny_llm {
 namespace detail {
@@ -93,21 +94,28 @@ __global__ __launch_bounds__(kCopyThreads) void kv_append_ranges_kernel(RangeArg
     *reinterpret_cast<uint4 *>(const_cast<__half *>(a.view.v_base) + dst) = v;
 }
 
-// Attended lengths and cache rows of a gather: in the kernel arguments up to
-// kGatherInline entries, so that the launch needs no metadata copy.
-constexpr int kGatherInline = 384;
 constexpr int kGatherPieces = 2; // 16-byte pieces per thread
 struct GatherArgs {
-    KvView         view;
-    const int32_t *lens; // device arrays (view.seq_row the rows), or null: the ones below
+    KvView         view; // seq_row: the cache rows
+    const int32_t *lens; // attended lengths
     int            Hkv;
     int            D;
     int            s_max;
     int            n;      // entries
     const __half  *src[2]; // what grid z counts: n entries of each output, K then V
     __half        *out[2];
-    int32_t        len[kGatherInline];
-    int32_t        row[kGatherInline];
+};
+
+// The first gather of a prepared step: lengths and rows in its arguments, up to
+// kGatherInline entries, so that it needs no metadata copy.  The 3 KB cost a
+// launch 0.4 us, so the kernel leaves them in device memory for the step's further
+// layers, which keep the small arguments (K of 3 sequences of 300 tokens: 6.8 us a
+// layer, 7.3 with the arrays in every launch).
+constexpr int kGatherInline = kGatherStore / 2;
+struct GatherStepArgs : GatherArgs {
+    int32_t *store; // [n lengths | n rows], or null
+    int32_t  len[kGatherInline];
+    int32_t  row[kGatherInline];
 };
 
 // grid (token blocks, Hkv, outputs * n): out[b][g][t][:] from the cache.  Two
@@ -120,13 +128,20 @@ struct GatherArgs {
 // three caches in turn 80.7 -> 68.2 us (5.9 TB/s read and written), over one 80.7
 // -> 52.8; 3 sequences of 300 tokens, where the metadata copy and the second
 // launch were most of it, 17.9 -> 10.7.
-template <bool STREAM>
-__global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
+// Args by value: through a reference they would be copied to scratch memory.
+template <bool STREAM, class Args>
+__device__ __forceinline__ void gather_body(Args a) {
     const int z = (int)blockIdx.z, which = z >= a.n, b = z - which * a.n;
     const int g = (int)blockIdx.y, blk = (int)blockIdx.x;
     const int ppt = a.D >> 3; // pieces per token
-    const int len = a.lens ? a.lens[b] : a.len[b];
-    const int row = a.lens ? (a.view.seq_row ? a.view.seq_row[b] : b) : a.row[b];
+    int       len, row;
+    if constexpr (std::is_same_v<Args, GatherStepArgs>) {
+        len = a.len[b];
+        row = a.row[b];
+    } else {
+        len = a.lens[b];
+        row = a.view.seq_row[b];
+    }
     const __half *const src = (which ? a.src[1] : a.src[0]) + (int64_t)g * a.view.head_stride;
     __half *const       out = (which ? a.out[1] : a.out[0]) + ((int64_t)b * a.Hkv + g) * a.s_max * a.D;
     uint4 val[kGatherPieces];
@@ -151,6 +166,21 @@ __global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
         if constexpr (STREAM) __builtin_nontemporal_store(__builtin_bit_cast(u32x4, val[u]), dst);
         else *dst = __builtin_bit_cast(u32x4, val[u]);
     }
+}
+
+template <bool STREAM>
+__global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
+    gather_body<STREAM>(a);
+}
+
+template <bool STREAM>
+__global__ __launch_bounds__(kCopyThreads) void kv_gather_step_kernel(GatherStepArgs a) {
+    gather_body<STREAM>(a);
+    if (a.store && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0)
+        for (int i = (int)threadIdx.x; i < a.n; i += kCopyThreads) {
+            a.store[i] = a.len[i];
+            a.store[a.n + i] = a.row[i];
+        }
 }
 
 struct TableArgs {
@@ -244,19 +274,23 @@ void launch_kv_append_ranges(const KvView &view, const int32_t *rows, const int3
 
 bool gather_inline(int n) { return n <= kGatherInline; }
 
-void launch_kv_gather(const KvView &view, const int32_t *lens, const int32_t *host_lens, const int32_t *host_rows, int n,
-                      int Hkv, int D, int s_max, __half *k_out, __half *v_out, hipStream_t stream) {
+void launch_kv_gather(const KvView &view, const GatherMeta &meta, int n, int Hkv, int D, int s_max, __half *k_out,
+                      __half *v_out, hipStream_t stream) {
     if (n <= 0 || s_max <= 0 || (!k_out && !v_out)) return;
-    GatherArgs a;
+    GatherStepArgs    a;
+    const GatherArgs &small = a;
+    const bool        inl = !meta.lens;
     a.view = view;
-    a.lens = gather_inline(n) ? nullptr : lens;
+    a.view.seq_row = meta.rows;
+    a.lens = meta.lens;
     a.Hkv = Hkv;
     a.D = D;
     a.s_max = s_max;
     a.n = n;
-    if (!a.lens) {
-        std::memcpy(a.len, host_lens, sizeof(int32_t) * (size_t)n);
-        std::memcpy(a.row, host_rows, sizeof(int32_t) * (size_t)n);
+    if (inl) {
+        std::memcpy(a.len, meta.host_lens, sizeof(int32_t) * (size_t)n);
+        std::memcpy(a.row, meta.host_rows, sizeof(int32_t) * (size_t)n);
+        a.store = meta.store;
     }
     const int64_t pieces = (int64_t)s_max * (D / 8), per = (int64_t)kCopyThreads * kGatherPieces;
     const int64_t blocks = (pieces + per - 1) / per;
@@ -264,10 +298,12 @@ void launch_kv_gather(const KvView &view, const int32_t *lens, const int32_t *ho
     auto          go = [&](int outputs) {
         const dim3 grid((unsigned)blocks, (unsigned)Hkv, (unsigned)(outputs * n));
         profile_begin(KernelId::KvGather, stream);
-        if (bytes > (32LL << 20))
-            hipLaunchKernelGGL((kv_gather_kernel<true>), grid, dim3(kCopyThreads), 0, stream, a);
-        else
-            hipLaunchKernelGGL((kv_gather_kernel<false>), grid, dim3(kCopyThreads), 0, stream, a);
+        const bool big = bytes > (32LL << 20);
+        const dim3 block(kCopyThreads);
+        if (inl && big) hipLaunchKernelGGL((kv_gather_step_kernel<true>), grid, block, 0, stream, a);
+        else if (inl) hipLaunchKernelGGL((kv_gather_step_kernel<false>), grid, block, 0, stream, a);
+        else if (big) hipLaunchKernelGGL((kv_gather_kernel<true>), grid, block, 0, stream, small);
+        else hipLaunchKernelGGL((kv_gather_kernel<false>), grid, block, 0, stream, small);
         HIP_CHECK(hipGetLastError());
         profile_end(KernelId::KvGather, stream);
     };

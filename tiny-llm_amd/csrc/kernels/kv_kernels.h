@@ -127,13 +127,22 @@ void launch_kv_append_ranges(const KvView &view, const int32_t *rows, const int3
                              const int32_t *counts, int n, int row_elems, const __half *new_k,
                              const __half *new_v, hipStream_t stream);
 
-// k_out / v_out (either may be null): out[b][g][t][:] = cache(b, g, t) for t <
-// len[b], +0.0 for len[b] <= t < s_max.  Lengths and cache rows of the n entries
-// come from host memory where gather_inline(n) (they travel in the kernel
-// arguments), else from the device arrays lens and view.seq_row.
+// Where a gather has its lengths and cache rows from: device arrays, or, with
+// `lens` null and gather_inline(n), host memory.  The launch then has them in its
+// arguments and leaves them in `store` (kGatherStore words of device memory, [n
+// lengths | n rows], may be null) for further launches.
+constexpr int kGatherStore = 768;
+struct GatherMeta {
+    const int32_t *lens = nullptr, *rows = nullptr;
+    const int32_t *host_lens = nullptr, *host_rows = nullptr;
+    int32_t       *store = nullptr;
+};
 bool gather_inline(int n);
-void launch_kv_gather(const KvView &view, const int32_t *lens, const int32_t *host_lens, const int32_t *host_rows, int n,
-                      int Hkv, int D, int s_max, __half *k_out, __half *v_out, hipStream_t stream);
+
+// k_out / v_out (either may be null): out[b][g][t][:] = cache(b, g, t) for t <
+// len[b], +0.0 for len[b] <= t < s_max.
+void launch_kv_gather(const KvView &view, const GatherMeta &meta, int n, int Hkv, int D, int s_max, __half *k_out,
+                      __half *v_out, hipStream_t stream);
 
 // Writes table[idx[i]] = val[i] for the n (index, value) pairs, in stream
 // order: the device copy of a block table follows its host mirror with only

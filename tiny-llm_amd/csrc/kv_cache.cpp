@@ -472,7 +472,7 @@ KvView KVCacheManager::layerView(int layer_idx, const int32_t *seq_row_dev) cons
 
 DecodeBatch::DecodeBatch(KVCacheManager &mgr, int max_seqs, int num_q_heads)
     : mgr_(mgr), max_seqs_(max_seqs), num_q_heads_(num_q_heads),
-      meta_(new detail::MetaRing(4, 2 * sizeof(int32_t) * detail::kDecRows)),
+      meta_(new detail::MetaRing(4, 2 * sizeof(int32_t) * detail::kDecRows, sizeof(int32_t) * detail::kGatherStore)),
       work_(new detail::Workspace()), gemm_work_(new detail::Workspace()),
       plan_(new detail::WorkList()),
       inl_(new detail::InlineMeta()) {}
@@ -513,7 +513,7 @@ Result<void> DecodeBatch::upload(const int *seq_ids, const int *attended, int n,
     // A failed prepare leaves an empty batch.
     n_ = 0;
     appendable_ = false;
-    d_rows_ = nullptr;
+    d_rows_ = d_gather_ = nullptr;
     ids_.clear();
     const KVCacheConfig &cfg = mgr_.getConfig();
     std::vector<char>    taken(static_cast<size_t>(cfg.max_batch_size), 0);
@@ -691,9 +691,26 @@ Result<void> DecodeBatch::gather(int layer_idx, half *k_out, half *v_out, int s_
         return Result<void>::err("DecodeBatch: Invalid layer_idx: " + std::to_string(layer_idx));
     if (s_max < 0) return Result<void>::err("DecodeBatch: s_max must be >= 0");
     if (n_ == 0 || s_max == 0) return Result<void>::ok();
-    if (!detail::gather_inline(n_)) upload_device(stream);
-    detail::launch_kv_gather(mgr_.layerView(layer_idx, d_slot_), d_lens_, lens_.data(), slot_.data(), n_, cfg.num_heads,
-                             cfg.head_dim, s_max, k_out, v_out, stream);
+    detail::GatherMeta meta;
+    if (uploaded_ || !detail::gather_inline(n_)) {
+        upload_device(stream);
+        meta.lens = d_lens_;
+        meta.rows = d_slot_;
+    } else if (d_gather_ && gather_stream_ == stream && !detail::stream_capturing(stream)) {
+        meta.lens = d_gather_;
+        meta.rows = d_gather_ + n_;
+    } else {
+        meta.host_lens = lens_.data();
+        meta.host_rows = slot_.data();
+        // (as in project: a captured launch carries what it needs)
+        if (!detail::stream_capturing(stream)) meta.store = meta_->next_tail(1);
+    }
+    detail::launch_kv_gather(mgr_.layerView(layer_idx, nullptr), meta, n_, cfg.num_heads, cfg.head_dim, s_max, k_out,
+                             v_out, stream);
+    if (meta.store) {
+        d_gather_ = meta.store;
+        gather_stream_ = stream;
+    }
     return Result<void>::ok();
 }
 
@@ -755,7 +772,7 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
         rows.seq_row = d_rows_;
         rows.wpos = d_rows_ + n_;
     } else {
-        store = rows.store = meta_->next_tail();
+        store = rows.store = meta_->next_tail(0);
     }
     detail::launch_w8a16(x, hidden, n_, hidden, group_size, segs, nseg, &rows, ws, stream, packed);
     if (store) {

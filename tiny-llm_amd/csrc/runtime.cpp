@@ -106,7 +106,7 @@ int32_t *DeviceRing::next() {
 }
 
 // ---------------------------------------------------------------- MetaRing
-MetaRing::MetaRing(int slots, size_t tail) : slots_(static_cast<size_t>(slots)), tail_(tail) {}
+MetaRing::MetaRing(int slots, size_t tail0, size_t tail1) : slots_(static_cast<size_t>(slots)), tails_{tail0, tail1} {}
 
 MetaRing::~MetaRing() {
     // kernels queued on callers' streams may still read the device slots
@@ -142,7 +142,7 @@ void MetaRing::grow(Slot &s, size_t bytes) {
     while (cap < bytes) cap <<= 1;
     void *host = nullptr, *dev = nullptr;
     HIP_CHECK(hipHostMalloc(&host, cap, hipHostMallocDefault));
-    HIP_CHECK(hipMalloc(&dev, cap + tail_));
+    HIP_CHECK(hipMalloc(&dev, cap + tails_[0] + tails_[1]));
     // The old host buffer is idle (its copy completed: begin() waited on the
     // slot's event); the old device buffer may still be read by queued kernels.
     if (s.host) retired_host_.push_back(s.host);
@@ -152,10 +152,11 @@ void MetaRing::grow(Slot &s, size_t bytes) {
     s.cap = cap;
 }
 
-int32_t *MetaRing::next_tail() {
-    tail_cur_ = (tail_cur_ + 1) % slots_.size();
-    const Slot &s = slots_[tail_cur_];
-    return reinterpret_cast<int32_t *>(static_cast<char *>(s.dev) + s.cap);
+int32_t *MetaRing::next_tail(int which) {
+    size_t &cur = tail_cur_[which];
+    cur = (cur + 1) % slots_.size();
+    const Slot &s = slots_[cur];
+    return reinterpret_cast<int32_t *>(static_cast<char *>(s.dev) + s.cap + (which ? tails_[0] : 0));
 }
 
 void MetaRing::reserve(size_t bytes) {

@@ -22,8 +22,9 @@ namespace detail {
 // memory next to the attention kernel and slowed it by more than it hid.)
 class MetaRing {
   public:
-    // tail: bytes behind each slot's device buffer for kernels to fill (next_tail).
-    explicit MetaRing(int slots = 4, size_t tail = 0);
+    // tail0, tail1: bytes of two areas behind each slot's device buffer for kernels
+    // to fill (next_tail).
+    explicit MetaRing(int slots = 4, size_t tail0 = 0, size_t tail1 = 0);
     ~MetaRing();
     MetaRing(const MetaRing &) = delete;
     MetaRing &operator=(const MetaRing &) = delete;
@@ -33,10 +34,10 @@ class MetaRing {
     // Sizes every slot for `bytes` now, so steps up to that size never
     // allocate.
     void reserve(size_t bytes);
-    // The tails in turn, after reserve(): what the first launch of a step brings
-    // in its arguments, kept for the step's further launches.  Ordered like the
-    // device buffers.
-    int32_t *next_tail();
+    // The slots' areas `which` in turn, after reserve(): what the first launch of a
+    // step brings in its arguments, kept for the step's further launches.  Ordered
+    // like the device buffers.
+    int32_t *next_tail(int which);
 
   private:
     struct Slot {
@@ -54,8 +55,8 @@ class MetaRing {
     std::vector<void *> retired_dev_, retired_host_;
     int                 cur_ = -1;
     size_t              bytes_ = 0;
-    const size_t        tail_;
-    size_t              tail_cur_ = 0;
+    const size_t        tails_[2];
+    size_t              tail_cur_[2] = {0, 0};
 };
 
 // Ring of four equal device buffers that kernels fill: what the first launch

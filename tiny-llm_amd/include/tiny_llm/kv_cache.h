@@ -218,6 +218,9 @@ class DecodeBatch {
     // memory, on rows_stream_, for the next ones (null: none has yet).
     const int32_t  *d_rows_ = nullptr;
     hipStream_t     rows_stream_ = nullptr;
+    // The same for its first gather: lengths and rows.
+    const int32_t  *d_gather_ = nullptr;
+    hipStream_t     gather_stream_ = nullptr;
 };
 
 // A prefill step over n sequences of one manager: sequence i brings

@@ -1,5 +1,6 @@
-"""GPU: the prompt-sized W8A16 kernel (more than 64 rows) at the edges of its
-tiles, K halves and scale groups, against the product in 64 bits.  Bar: 1e-3
+"""GPU: W8A16 products of more than 64 rows, in the prompt-sized kernel at the
+edges of its tiles, K halves and scale groups and in the split-K kernel beside
+it, against the product in 64 bits.  Bar: 1e-3
 normwise per row, the W8A16 bar (fp16 rounding of an output leaves 2^-11)."""
 import numpy as np
 import pytest
@@ -26,6 +27,8 @@ def product(x, w, s, K, gs):
     return x.view(np.float16).astype(np.float64) @ (w.astype(np.float64) * sc)
 
 
+# Shapes at the edges of both kernels' tiles; which runs each is the planner's
+# choice (TILE_SHAPES states it).
 @pytest.mark.parametrize("M,N,K,gs", [
     (65, 36304, 32, 32),     # one row over, one k step: no chunk at all, a column tail
     (127, 18608, 64, 64),    # one chunk of two steps: the second K half is empty
@@ -36,7 +39,7 @@ def product(x, w, s, K, gs):
     (200, 6560, 2080, 512),  # few rows with a long K; groups across chunks and the K halves' boundary
     (2390, 1008, 192, 256),  # more row tiles than a panel, a group longer than K
     (9250, 256, 64, 32),     # one column tile
-    (600, 8192, 1056, 128),  # the widest tiles' other shapes
+    (600, 8192, 1056, 128),  # 128 x 192 tiles
 ])
 def test_w8a16_tile_edges(tl, orc, M, N, K, gs):
     rng = np.random.default_rng(M + 3 * N + 7 * K + gs)
@@ -156,7 +159,7 @@ def test_w8a16_tile_unaligned_output(tl, orc):
 
 
 def test_w8a16_tile_element_stores(tl, orc):
-    """As above where the tile kernel writes the outputs."""
+    """The same in the tile kernel."""
     M, N, K, gs = 585, 8208, 160, 128
     assert tl.w8a16_plan(M, N, K, gs)[0] == "tile"
     rng = np.random.default_rng(14)

@@ -1,4 +1,4 @@
-// The reference's attention-weights and softmax kernels for gfx950
+// The reference's test-side attention-weights and softmax kernels for gfx950
 // (get_attention_weights and softmax, attention.cu:240-343).
 #include "prefill.h"
 

@@ -125,7 +125,7 @@ struct GatherStepArgs : GatherArgs {
 // reader: they no longer evict what is still to be read.  (Non-temporal loads
 // too: 68 us where this takes 53.)  Bound by memory: 16 ragged sequences of up
 // to 4096 tokens from 16-token blocks, 8 heads of 128, prepare + gather over
-// three caches in turn 80.7 -> 68.2 us (5.9 TB/s read and written), over one 80.7
+// three caches in turn 81.0 -> 65.8 us (6.1 TB/s read and written), over one 80.7
 // -> 52.8; 3 sequences of 300 tokens, where the metadata copy and the second
 // launch were most of it, 17.9 -> 10.7.
 // Args by value: through a reference they would be copied to scratch memory.

@@ -1,7 +1,7 @@
 // Launch interface of the prefill-side attention kernels (gfx950):
 // causal attention of new query tokens over a KV view (the cache-native
 // prefill, and the reference's compact attention_prefill), plus the
-// reference's softmax and attention-weights kernels.
+// reference's test-side softmax and attention-weights kernels.
 #pragma once
 
 #include "kv_kernels.h"

@@ -58,6 +58,8 @@ def test_tile_shape_by_the_time_of_its_rounds(tl):
     three rounds of it (68 against 70)."""
     assert plan(tl, 1536, 4096, 4096) == ("tile", 128, 256)
     assert plan(tl, 1536, 4096, 4096, packed=True) == ("tile", 64, 128)
+    # groups of 32 leave no room for two: 155 us, 197 in sixteen rounds of the smallest
+    assert plan(tl, 4096, 8192, 1024, 32, packed=True) == ("tile", 128, 192)
 
 
 def test_kernel_by_size_alone(tl):

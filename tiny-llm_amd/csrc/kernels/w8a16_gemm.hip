@@ -1531,11 +1531,11 @@ struct TilePlan {
 // 128: 64 x 128 / 192 / 256 tiles 34 / 47 / 58 us row-major and 28 / 38 / 46
 // packed, 128 x 128 / 192 / 256 48 / 64 / 77 and 43 / 56 / 70.  Two packed 64 x 128
 // workgroups fit a CU, so that their further rounds add 20 us, not 28.  Groups of
-// 32 rescale twice a chunk and take a third more.
+// 32 rescale twice a chunk, take a third more, and leave no room for that.
 float tile_us(int rb, int cb, int64_t rounds, int K, int gs, bool packed) {
     static constexpr float kNs[2][2][3] = {{{6.9f, 9.4f, 11.8f}, {9.8f, 12.9f, 15.6f}},
                                            {{5.7f, 7.7f, 9.4f}, {8.6f, 11.3f, 14.2f}}};
-    const float r = packed && rb == 4 && cb == 2 ? 0.3f + 0.7f * (float)rounds : (float)rounds;
+    const float r = packed && rb == 4 && cb == 2 && gs > 32 ? 0.3f + 0.7f * (float)rounds : (float)rounds;
     return r * kNs[packed][rb / 4 - 1][cb - 2] * 1e-3f * (float)(K + 850) * (gs == 32 ? 1.3f : 1.0f);
 }
 
@@ -1561,8 +1561,8 @@ TilePlan tile_plan(int M, int K, int gs, const W8A16Seg *segs, int nseg, bool pa
 // weights, where the two kernels are nearest.  The split-K kernel takes 2.2 us + K *
 // 2.65 ns for each 64 x 64 tile that a CU gets, whole tiles, and up to 256 rows,
 // where K is split and partials are written and summed, 2.5 us + K * 4.7 ns per
-// tile and CU (groups below 128, with their second accumulator, 10 and 25%
-// more).  The margin is for row-major weights, which lose more with a short K, and
+// tile and CU (with the second accumulator of groups of 64 and 32 10 and 20%
+// more, split 25%).  The margin is for row-major weights, which lose more with a short K, and
 // with groups of 32 up to 256 rows.
 //
 // Measured on 2900 products (K 512 .. 14336, 80 .. 4096 rows, both layouts) and 378
@@ -1571,15 +1571,15 @@ TilePlan tile_plan(int M, int K, int gs, const W8A16Seg *segs, int nseg, bool pa
 // replace, made 146 products slower, by up to 40% (1152 x 8192 x 512 row-major 33
 // -> 46 us), and 34 projections, whose k and v parts stay with the split-K kernel in
 // a second launch, by up to 38% (1152 x (2048 + 2 x 256) x 2048 row-major 31 -> 43).
-// These make no product slower, and 9 projections, by up to 15% (1152 x
-// (4096 + 2 x 512) x 2048 row-major 50 -> 57; the q part alone 48 -> 37): a rule that
-// spares those too leaves 13% of the products at up to twice their time.
+// These make no product slower by more than 3%, and 9 projections, by up to 12%
+// (1152 x (4096 + 2 x 1024) x 4096 packed 91 -> 102; the q part alone 70 -> 56): a
+// rule that spares those too leaves 13% of the products at up to twice their time.
 bool tile_ok(int M, int K, int gs, const W8A16Seg &seg, int cus) {
     if (M <= kDecRows) return false;
     const float tiles = (float)((M + kBM - 1) / kBM) * (float)((seg.n + kBN - 1) / kBN) / (float)cus;
     const bool  split = M <= 256 && K >= 1024;
     const float sk = split ? (tiles + 0.2f) * (2.5f + 4.7e-3f * (float)K) * (gs < 128 ? 1.25f : 1.0f)
-                           : std::ceil(tiles) * (2.2f + 2.65e-3f * (float)K) * (gs < 128 ? 1.1f : 1.0f);
+                           : std::ceil(tiles) * (2.2f + 2.65e-3f * (float)K) * (gs == 32 ? 1.2f : gs == 64 ? 1.1f : 1.0f);
     const float bar = sk / (K < 1024 || (split && gs == 32) ? 1.2f : 1.08f);
     if (tile_us(4, 2, 1, K, gs, true) > bar) return false; // (the least there is: no plan for small products)
     return tile_plan(M, K, gs, &seg, 1, true, cus).us <= bar;

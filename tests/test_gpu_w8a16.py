@@ -336,6 +336,42 @@ def test_project_replays_under_hip_graph_capture(tl, orc):
     del graph
 
 
+def test_captured_step_after_an_append_keeps_its_rows(tl, orc):
+    """A projection and a gather that are captured after an append of the same
+    step, whose metadata is then on the device already, replay with that step's
+    rows after further steps have rewritten every device buffer."""
+    L, Hkv, G, D, hidden, gs, n = 1, 2, 4, 64, 256, 64, 9
+    g, _, ids, keep = _cache(tl, orc, np.random.default_rng(14), L, Hkv, D, 96, list(range(1, n + 1)), False)
+    rng = np.random.default_rng(16)
+    fused, separate = _layer_projections(tl, orc, rng, L, Hkv, G, D, hidden, gs)
+    dx, noise = (to_dev(orc.f2h(rng.standard_normal((n, hidden)).astype(np.float32))) for _ in range(2))
+    kv = to_dev(orc.f2h(rng.standard_normal((n, Hkv * D)).astype(np.float32)))
+    batch, out = tl.DecodeBatch(g, n, Hkv * G), empty_dev((2, n, Hkv, 16, D))
+
+    def step():
+        fused(batch, 0, dx, stream())
+        batch.gather(0, out[0].data_ptr(), out[1].data_ptr(), 16, stream())
+
+    batch.prepare(ids, stream())
+    batch.append(0, 1, kv.data_ptr(), kv.data_ptr(), stream())
+    step()
+    elems = g.slot_bytes() // 2 * (n + 1)
+    want, want_out = read_dev(g.pool(), elems), to_host(out)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for rep in range(3):
+        for i in range(5):  # other rows through every device buffer, over the same positions
+            batch.prepare([ids[j] for j in np.roll(np.arange(n), 1 + i + rep)], stream())
+            batch.append(0, 1, kv.data_ptr(), kv.data_ptr(), stream())
+            fused(batch, 0, noise, stream())
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        assert np.array_equal(read_dev(g.pool(), elems), want) and np.array_equal(to_host(out), want_out), rep
+    del graph
+
+
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("paged", [False, True])
 def test_project_fused_append(tl, orc, paged, packed):

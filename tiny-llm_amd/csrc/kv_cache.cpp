@@ -692,18 +692,19 @@ Result<void> DecodeBatch::gather(int layer_idx, half *k_out, half *v_out, int s_
     if (s_max < 0) return Result<void>::err("DecodeBatch: s_max must be >= 0");
     if (n_ == 0 || s_max == 0) return Result<void>::ok();
     detail::GatherMeta meta;
-    if (uploaded_ || !detail::gather_inline(n_)) {
+    const bool inl = detail::gather_inline(n_);
+    const bool captured = inl && detail::stream_capturing(stream); // (as in project)
+    if (!captured && (uploaded_ || !inl)) {
         upload_device(stream);
         meta.lens = d_lens_;
         meta.rows = d_slot_;
-    } else if (d_gather_ && gather_stream_ == stream && !detail::stream_capturing(stream)) {
+    } else if (!captured && d_gather_ && gather_stream_ == stream) {
         meta.lens = d_gather_;
         meta.rows = d_gather_ + n_;
     } else {
         meta.host_lens = lens_.data();
         meta.host_rows = slot_.data();
-        // (as in project: a captured launch carries what it needs)
-        if (!detail::stream_capturing(stream)) meta.store = meta_->next_tail(1);
+        if (!captured) meta.store = meta_->next_tail(1);
     }
     detail::launch_kv_gather(mgr_.layerView(layer_idx, nullptr), meta, n_, cfg.num_heads, cfg.head_dim, s_max, k_out,
                              v_out, stream);
@@ -761,13 +762,14 @@ Result<void> DecodeBatch::project(int layer_idx, const half *x, int hidden, int 
         return Result<void>::err("DecodeBatch: packed weights need hidden % 32 == 0 and group_size "
                                  "in {32, 64, 128, 256, 512}");
     int32_t *store = nullptr;
-    if (uploaded_ || !detail::w8a16_takes_dec(x, hidden, n_, hidden, group_size, segs, nseg, packed)) {
+    const bool dec = detail::w8a16_takes_dec(x, hidden, n_, hidden, group_size, segs, nseg, packed);
+    if (dec && detail::stream_capturing(stream)) {
+        // A captured launch keeps its rows in its arguments: replays then depend
+        // on nothing that later steps rewrite.
+    } else if (uploaded_ || !dec) {
         upload_device(stream); // (the other kernels read the rows from device memory)
         rows.seq_row = d_slot_;
         rows.wpos = d_wpos_;
-    } else if (detail::stream_capturing(stream)) {
-        // A captured launch keeps its rows in its arguments: replays then depend
-        // on nothing that later steps rewrite.
     } else if (d_rows_ && rows_stream_ == stream) {
         rows.seq_row = d_rows_;
         rows.wpos = d_rows_ + n_;
